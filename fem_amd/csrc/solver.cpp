@@ -641,12 +641,13 @@ void Context::build_hierarchy() {
     if (o.autotune) autotune<double>(h64);
     build_ops<double>(h64);
     h64_ops = true;
-    if (o.precond == FEMH_PRECOND_MG) {
+    // (a grid with an odd edge has one level: Jacobi, no smoother)
+    if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
       estimate_lmax(h64);
       upload_cheb(h64);
       // the coarsest level is inverted densely when it is small enough, else
       // solved approximately by a long Chebyshev polynomial (cheb_run)
-      if (nlevels > 1) dense_coarse(h64);
+      dense_coarse(h64);
     }
   } else {
     // mixed precision: the smoothing hierarchy is built in FP32 directly;
@@ -656,20 +657,18 @@ void Context::build_hierarchy() {
     launch_convert<double, float>(576, Ke64.as<double>(), h32.Ke.as<float>(), stream);
     if (o.autotune) autotune<float>(h32);
     build_ops<float>(h32);
-    if (o.precond == FEMH_PRECOND_MG) {
-      if (nlevels > 1) {
-        // dense coarsest inverse of the FP32 coarsest operator (host Cholesky
-        // in FP64 on its widened copy)
-        const Level<float> &Lc = h32.lv.back();
-        launch_convert<float, double>((size_t)243 * nb * Lc.g.V, Lc.S.as<float>(), h64.lv.back().S.as<double>(),
-                                      stream);
-        dense_coarse(h64);
-        if (h64.ndense) {
-          h32.Ainv.alloc(sizeof(float) * (size_t)h64.ndense * h64.ndense * B);
-          launch_convert<double, float>((size_t)h64.ndense * h64.ndense * nb, h64.Ainv.as<double>(),
-                                        h32.Ainv.as<float>(), stream);
-          h32.ndense = h64.ndense;
-        }
+    if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
+      // dense coarsest inverse of the FP32 coarsest operator (host Cholesky
+      // in FP64 on its widened copy)
+      const Level<float> &Lc = h32.lv.back();
+      launch_convert<float, double>((size_t)243 * nb * Lc.g.V, Lc.S.as<float>(), h64.lv.back().S.as<double>(),
+                                    stream);
+      dense_coarse(h64);
+      if (h64.ndense) {
+        h32.Ainv.alloc(sizeof(float) * (size_t)h64.ndense * h64.ndense * B);
+        launch_convert<double, float>((size_t)h64.ndense * h64.ndense * nb, h64.Ainv.as<double>(),
+                                      h32.Ainv.as<float>(), stream);
+        h32.ndense = h64.ndense;
       }
       estimate_lmax(h32);
       upload_cheb(h32);
@@ -685,8 +684,10 @@ void Context::ensure_h64_ops() {
   if (h64_ops) return;
   build_ops<double>(h64);
   // (spectrum bounds stay those of the FP32 operators)
-  if (o.precond == FEMH_PRECOND_MG && nlevels > 1) dense_coarse(h64);
-  if (o.precond == FEMH_PRECOND_MG) upload_cheb(h64);
+  if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
+    dense_coarse(h64);
+    upload_cheb(h64);
+  }
   h64_ops = true;
 }
 
