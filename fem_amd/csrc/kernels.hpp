@@ -124,6 +124,13 @@ void launch_restrict(Dims fine, Dims coarse, int R, const T *rf, T *rc, const in
 template <typename T>
 void launch_prolong_add(Dims fine, Dims coarse, int R, const T *ec, T *ef, const int *act,
                         hipStream_t s, T *out = nullptr, int planes = 0);
+// Ainv[s] = (A + (mean diagonal / V) Z Z^T)^-1 of each sample's operator with
+// stencil S on grid g (Z the three constant fields), formed in FP64;
+// bad[s] = 1 where a pivot was not positive (dense.hip).  work holds
+// dense_work_doubles(3 g.V, samples) doubles.
+size_t dense_work_doubles(int n, int B);
+template <typename T>
+void launch_dense_inverse(const Dims &g, int nb, const T *S, double *work, T *Ainv, int *bad, hipStream_t s);
 // dense coarsest solve: x = Ainv[s] b for each RHS (n = 3*V_coarsest)
 template <typename T>
 void launch_dense_solve(int n, int R, const T *Ainv, const T *b, T *x, const int *act,

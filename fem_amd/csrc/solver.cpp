@@ -432,72 +432,25 @@ void Context::estimate_lmax(Hierarchy<T> &h) {
 
 // Dense inverse of each sample's regularised coarsest operator A + s Z Z^T
 // (Z = the three constant displacement fields): for right-hand sides
-// orthogonal to Z it returns the zero-mean solution of A x = b.
-void Context::dense_coarse(Hierarchy<double> &h) {
-  Level<double> &L = h.lv.back();
-  const int V = L.g.V, n = 3 * V;
+// orthogonal to Z it returns the zero-mean solution of A x = b.  Formed on
+// the device in FP64 (dense.hip).
+template <typename T>
+void Context::dense_coarse(Hierarchy<T> &h) {
+  Level<T> &L = h.lv.back();
+  const int n = 3 * L.g.V;
   h.ndense = 0;
   if (n > 648 || h.lv.size() < 2) return;
-  std::vector<double> Sh((size_t)243 * V * nb);
-  FEMH_HIP(hipMemcpyAsync(Sh.data(), L.S.p, sizeof(double) * Sh.size(), hipMemcpyDeviceToHost, stream));
+  h.Ainv.alloc(sizeof(T) * (size_t)n * n * B);
+  dense_work.alloc(sizeof(double) * dense_work_doubles(n, B));
+  dense_bad.alloc(sizeof(int) * kMaxB);
+  launch_dense_inverse<T>(L.g, nb, L.S.template as<T>(), dense_work.as<double>(), h.Ainv.template as<T>(),
+                          dense_bad.as<int>(), stream);
+  FEMH_HIP(hipGetLastError());
+  int bad[kMaxB];
+  FEMH_HIP(hipMemcpyAsync(bad, dense_bad.p, sizeof(int) * nb, hipMemcpyDeviceToHost, stream));
   FEMH_HIP(hipStreamSynchronize(stream));
-  std::vector<double> inv((size_t)n * n * nb);
-  std::vector<double> A((size_t)n * n), col(n);
-  const Dims &d = L.g;
-  for (int smp = 0; smp < nb; smp++) {
-    const double *S = Sh.data() + (size_t)smp * 243 * V;
-    std::fill(A.begin(), A.end(), 0.0);
-    for (int N = 0; N < V; N++) {
-      const int k = N % d.nz, j = (N / d.nz) % d.ny, i = N / (d.nz * d.ny);
-      for (int off = 0; off < 27; off++) {
-        const int ni = (i + off / 9 - 1 + d.nx) % d.nx, nj = (j + (off / 3) % 3 - 1 + d.ny) % d.ny,
-                  nk = (k + off % 3 - 1 + d.nz) % d.nz;
-        const int M = (ni * d.ny + nj) * d.nz + nk;
-        for (int c = 0; c < 3; c++)
-          for (int dd = 0; dd < 3; dd++)
-            A[(size_t)(c * V + N) * n + dd * V + M] += S[stencil_index(off, 3 * c + dd, V, N)];
-      }
-    }
-    double dmean = 0;
-    for (int t = 0; t < n; t++) dmean += A[(size_t)t * n + t];
-    dmean /= n;
-    for (int c = 0; c < 3; c++)
-      for (int a = 0; a < V; a++)
-        for (int bb = 0; bb < V; bb++) A[(size_t)(c * V + a) * n + c * V + bb] += dmean / V;
-    // Cholesky A = L L^T (lower, in place)
-    for (int j = 0; j < n; j++) {
-      double s = A[(size_t)j * n + j];
-      for (int k = 0; k < j; k++) s -= A[(size_t)j * n + k] * A[(size_t)j * n + k];
-      if (!(s > 0)) throw Error(FEMH_NONFINITE, "coarsest operator is not positive definite");
-      s = std::sqrt(s);
-      A[(size_t)j * n + j] = s;
-      for (int i = j + 1; i < n; i++) {
-        double t = A[(size_t)i * n + j];
-        for (int k = 0; k < j; k++) t -= A[(size_t)i * n + k] * A[(size_t)j * n + k];
-        A[(size_t)i * n + j] = t / s;
-      }
-    }
-    double *Ai = inv.data() + (size_t)smp * n * n;
-    for (int c = 0; c < n; c++) {
-      std::fill(col.begin(), col.end(), 0.0);
-      col[c] = 1.0;
-      for (int i = 0; i < n; i++) {
-        double s = col[i];
-        for (int k = 0; k < i; k++) s -= A[(size_t)i * n + k] * col[k];
-        col[i] = s / A[(size_t)i * n + i];
-      }
-      for (int i = n - 1; i >= 0; i--) {
-        double s = col[i];
-        for (int k = i + 1; k < n; k++) s -= A[(size_t)k * n + i] * col[k];
-        col[i] = s / A[(size_t)i * n + i];
-      }
-      for (int i = 0; i < n; i++) Ai[(size_t)i * n + c] = col[i];
-    }
-  }
-  h.Ainv.alloc(sizeof(double) * (size_t)n * n * B);
-  FEMH_HIP(hipMemcpyAsync(h.Ainv.p, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice,
-                          stream));
-  FEMH_HIP(hipStreamSynchronize(stream));
+  for (int smp = 0; smp < nb; smp++)
+    if (bad[smp]) throw Error(FEMH_NONFINITE, "coarsest operator is not positive definite");
   h.ndense = n;
 }
 
@@ -658,18 +611,7 @@ void Context::build_hierarchy() {
     if (o.autotune) autotune<float>(h32);
     build_ops<float>(h32);
     if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
-      // dense coarsest inverse of the FP32 coarsest operator (host Cholesky
-      // in FP64 on its widened copy)
-      const Level<float> &Lc = h32.lv.back();
-      launch_convert<float, double>((size_t)243 * nb * Lc.g.V, Lc.S.as<float>(), h64.lv.back().S.as<double>(),
-                                    stream);
-      dense_coarse(h64);
-      if (h64.ndense) {
-        h32.Ainv.alloc(sizeof(float) * (size_t)h64.ndense * h64.ndense * B);
-        launch_convert<double, float>((size_t)h64.ndense * h64.ndense * nb, h64.Ainv.as<double>(),
-                                      h32.Ainv.as<float>(), stream);
-        h32.ndense = h64.ndense;
-      }
+      dense_coarse(h32);
       estimate_lmax(h32);
       upload_cheb(h32);
       for (int l = 0; l < nlevels; l++) h64.lv[l].lmax = h32.lv[l].lmax;

@@ -155,6 +155,7 @@ struct Context {
   // PCG iteration state on the device: iterations, state (int [kMaxR] each),
   // relative residual and |b|^2 (double [kMaxR] each)
   DBuf pcg_state;
+  DBuf dense_work, dense_bad;  // dense coarsest inverse: FP64 matrices and panels, per-sample failure flag
   DBuf ls_part, ls_h;  // device line search: per-cell block partials [n][kRedBlocks], steps [n]
   // recorded PCG iteration pairs (hipGraph), keyed by everything their
   // launches bake in: precision, right-hand sides, vector and hierarchy
@@ -280,7 +281,8 @@ struct Context {
   int residual_dots(const int *act_);
   template <typename T>
   void estimate_lmax(Hierarchy<T> &h);
-  void dense_coarse(Hierarchy<double> &h);
+  template <typename T>
+  void dense_coarse(Hierarchy<T> &h);
   void read_scalars(int slot, double *out, int n, int np);
   void compute_ch(const double *fields, double *C);
 };
