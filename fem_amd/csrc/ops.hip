@@ -45,29 +45,35 @@ constexpr int kEOH = 13;         // LDS stride of one voxel's 12 plane forces (o
 __device__ __forceinline__ int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 // epilogue inputs of one owned node (loaded ahead of the operator work so
-// that their latency overlaps it):
-//   EP_RES: e0 = b ; EP_CHEB0: e0 = b, e1 = 1/D ; EP_STEP: e0 = rprev, e1 = 1/D,
-//   e2 = xprev (0 without one)
+// that their latency overlaps it; the set of loads is fixed per variant -- a
+// load behind a run-time branch is waited for at the branch's end):
+//   EP_RES, EP_PRE: e0 = b ; EP_CHEB0, EP_CHEB0L, EP_FIN1: e0 = b, e1 = 1/D ;
+//   EP_STEP, EP_LAST, EP_LASTD: e0 = rprev, e1 = 1/D, e2 = xprev (none from a
+//   zero start, ST_DSCALE) ; EP_LASTD: e3 = b (for b . x) ; EP_AXD: e1 = 1/D
 template <typename T>
 struct EpiIn {
-  T e0[3], e1[3], e2[3], e3[3];  // e3: EP_STEP with a dot: b (for b . x)
+  T e0[3], e1[3], e2[3], e3[3];
 };
+__host__ __device__ constexpr bool ep_is_step(int ep) { return ep == EP_STEP || ep == EP_LAST || ep == EP_LASTD; }
+__host__ __device__ constexpr bool ep_has_b(int ep) {
+  return ep == EP_RES || ep == EP_PRE || ep == EP_CHEB0 || ep == EP_CHEB0L || ep == EP_FIN1;
+}
 
-template <typename T, int EP>
+template <typename T, int ST, int EP>
 __device__ __forceinline__ void epi_load(const OpArgs<T> &a, const T *__restrict__ Ds, size_t off,
                                          int V, int n, EpiIn<T> &p) {
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     const size_t q = off + (size_t)c * V + n;
-    if (EP == EP_RES || EP == EP_CHEB0) p.e0[c] = a.b[q];
-    if (EP == EP_STEP) p.e0[c] = a.rprev[q];
-    if (EP == EP_CHEB0 || EP == EP_STEP || (EP == EP_AX && a.ydinv)) p.e1[c] = Ds[(size_t)c * V + n];
-    if (EP == EP_STEP) p.e2[c] = a.xprev ? a.xprev[q] : (T)0;
-    if (EP == EP_STEP) p.e3[c] = a.dot ? a.b[q] : (T)0;
+    if (ep_has_b(EP)) p.e0[c] = a.b[q];
+    if (ep_is_step(EP)) p.e0[c] = a.rprev[q];
+    if (EP == EP_CHEB0 || EP == EP_FIN1 || ep_is_step(EP) || EP == EP_AXD) p.e1[c] = Ds[(size_t)c * V + n];
+    if (ep_is_step(EP)) p.e2[c] = ST == ST_DSCALE ? (T)0 : a.xprev[q];
+    if (EP == EP_LASTD) p.e3[c] = a.b[q];
   }
 }
 
-// FP64 partial sums of the epilogue: EP_AX u.Au ; EP_STEP b.x_new ;
+// FP64 partial sums of the epilogue: EP_AX u.Au ; EP_FIN1, EP_LASTD b.x_new ;
 // EP_RES r.r, b.x, x.r (x = the staged vector)
 struct DotAcc {
   double a = 0, b = 0, c = 0;
@@ -85,7 +91,7 @@ __device__ __forceinline__ void ep_store(T *p, T v) {
 }
 
 // epilogue at one owned node (all three components)
-template <typename T, int EP, bool NT = false>
+template <typename T, int ST, int EP, bool NT = false>
 __device__ __forceinline__ void epilogue(const OpArgs<T> &a, const EpiIn<T> &p, T ti, T c1, T c2,
                                          size_t off, int V, int n, const T Au[3], const T uo[3],
                                          DotAcc &dv) {
@@ -93,40 +99,41 @@ __device__ __forceinline__ void epilogue(const OpArgs<T> &a, const EpiIn<T> &p, 
   for (int c = 0; c < 3; c++) {
     const size_t q = off + (size_t)c * V + n;
     if (EP == EP_AX) {
-      ep_store<NT>(&a.y[q], a.ydinv ? Au[c] * p.e1[c] : Au[c]);
-      if (a.pout) ep_store<NT>(&a.pout[q], uo[c]);
+      ep_store<NT>(&a.y[q], Au[c]);
+      if (ST == ST_PUPD) ep_store<NT>(&a.pout[q], uo[c]);
       if (a.dot) dv.a += (double)uo[c] * (double)Au[c];
-    } else if (EP == EP_RES) {
+    } else if (EP == EP_AXD) {
+      ep_store<NT>(&a.y[q], Au[c] * p.e1[c]);
+    } else if (EP == EP_RES || EP == EP_PRE) {
       const T rv = p.e0[c] - Au[c];
       ep_store<NT>(&a.y[q], rv);
-      if (a.dot) {
+      if (EP == EP_RES && a.dot) {
         dv.a += (double)rv * (double)rv;
         dv.b += (double)p.e0[c] * (double)uo[c];
         dv.c += (double)uo[c] * (double)rv;
       }
-    } else if (EP == EP_CHEB0) {
+    } else if (EP == EP_FIN1) {
       const T rv = p.e0[c] - Au[c];
-      if (a.fin1) {
-        const T xv = uo[c] + rv * ti * p.e1[c];
-        ep_store<NT>(&a.x[q], xv);
-        if (a.dot) dv.a += (double)p.e0[c] * (double)xv;
-      } else {
-        ep_store<NT>(&a.r[q], rv);
-        if (!a.last) ep_store<NT>(&a.dout[q], rv * ti * p.e1[c]);  // `last`: no smoothing step follows
-        ep_store<NT>(&a.x[q], uo[c]);
-      }
-    } else {  // EP_STEP
+      const T xv = uo[c] + rv * ti * p.e1[c];
+      ep_store<NT>(&a.x[q], xv);
+      if (a.dot) dv.a += (double)p.e0[c] * (double)xv;
+    } else if (EP == EP_CHEB0 || EP == EP_CHEB0L) {
+      const T rv = p.e0[c] - Au[c];
+      ep_store<NT>(&a.r[q], rv);
+      if (EP == EP_CHEB0) ep_store<NT>(&a.dout[q], rv * ti * p.e1[c]);
+      ep_store<NT>(&a.x[q], uo[c]);
+    } else {
       const T rv = p.e0[c] - Au[c];
       const T dn = c1 * uo[c] + c2 * rv * p.e1[c];
       T xv = p.e2[c] + uo[c];
-      if (a.last) {
+      if (EP != EP_STEP) {
         xv += dn;  // the last step's r and d are not read again
       } else {
         ep_store<NT>(&a.r[q], rv);
         ep_store<NT>(&a.dout[q], dn);
       }
       ep_store<NT>(&a.x[q], xv);
-      if (a.dot) dv.a += (double)p.e3[c] * (double)xv;
+      if (EP == EP_LASTD) dv.a += (double)p.e3[c] * (double)xv;
     }
   }
 }
@@ -173,16 +180,21 @@ static inline int tiled_tiles(const Dims &g, const TileShape &ts) {
 
 static int tiled_resident(int sz, const TileShape &ts);
 
+// Launches with a fused grid transfer (`fused`) have chunks of an even length,
+// so that a chunk holds whole coarse planes; the others may take odd ones (a
+// 16^3 cell: one plane per workgroup).
+static inline int even_chunk(int ti, bool fused) { return fused ? ti + (ti & 1) : ti; }
+
 // Chunk length for a launch whose active workgroups (Ract active right-hand
 // sides) fill the device about once or less: the rounds of resident
 // workgroups set the time, so take the length that minimises rounds x slabs
 // per workgroup (at most 255 planes, the width of the launch-shape field).
-static int round_chunk(const Dims &g, const TileShape &ts, int tiles, int Ract, int sz) {
+static int round_chunk(const Dims &g, const TileShape &ts, int tiles, int Ract, int sz, bool fused = false) {
   const long res = tiled_resident(sz, ts);
   long best = LONG_MAX;
   int TI = g.nx;
-  for (int c = (g.nx + 254) / 255; c <= g.nx; c++) {
-    const int ti = (g.nx + c - 1) / c, ch = (g.nx + ti - 1) / ti;
+  for (int c = (g.nx + 253) / 254; c <= g.nx; c++) {
+    const int ti = even_chunk((g.nx + c - 1) / c, fused), ch = (g.nx + ti - 1) / ti;
     if ((long)tiles * ch > kMaxPartials) continue;
     const long rounds = ((long)tiles * ch * Ract + res - 1) / res, cost = rounds * (ti + 1);
     if (cost < best) {
@@ -193,7 +205,7 @@ static int round_chunk(const Dims &g, const TileShape &ts, int tiles, int Ract, 
   return TI;
 }
 
-static inline int tiled_chunk(const Dims &g, int R, int shape, int sz) {
+static inline int tiled_chunk(const Dims &g, int R, int shape, int sz, bool fused = false) {
   const TileShape ts = tile_of(g, R, shape);
   const int tiles = tiled_tiles(g, ts);
   const int want = shape & 0xff;
@@ -210,12 +222,13 @@ static inline int tiled_chunk(const Dims &g, int R, int shape, int sz) {
   if (want > 0) {
     TI = want;
   } else if (R <= kRHS) {
-    TI = round_chunk(g, ts, tiles, R, sz);
+    TI = round_chunk(g, ts, tiles, R, sz, fused);
   } else {
     while (TI > 2 && (long)tiles * ((g.nx + TI - 1) / TI) * R * ts.tj * ts.tk < 512L * 256) TI /= 2;
   }
   if (TI > g.nx) TI = g.nx;
-  while ((long)tiles * ((g.nx + TI - 1) / TI) > kMaxPartials) TI++;
+  TI = even_chunk(TI, fused);
+  while ((long)tiles * ((g.nx + TI - 1) / TI) > kMaxPartials) TI = even_chunk(TI + 1, fused);
   return TI;
 }
 
@@ -229,8 +242,8 @@ int tiled_sparse_shape(const Dims &g, int R, int Ract, int shape, int sz) {
   return tiled_shape_code(v, round_chunk(g, ts, tiled_tiles(g, ts), Ract, sz));
 }
 
-int tiled_parts(const Dims &g, int R, int shape, int sz) {
-  const int TI = tiled_chunk(g, R, shape, sz);
+int tiled_parts(const Dims &g, int R, int shape, int sz, bool fused) {
+  const int TI = tiled_chunk(g, R, shape, sz, fused);
   return tiled_tiles(g, tile_of(g, R, shape)) * ((g.nx + TI - 1) / TI);
 }
 
@@ -268,24 +281,43 @@ __device__ __forceinline__ double bload(__amdgpu_buffer_rsrc_t r, unsigned voff,
 // overwritten two slabs after it was filled, behind the barrier that closes
 // the slab in between (every read of it -- the FP64 bottom face, the owned
 // node's staged value -- happens before that barrier).
-// Waves per SIMD the FP32 variants are compiled for: 4 (at most 128 VGPRs),
-// except the D^-1-scaled Chebyshev step (two smoothing steps in one launch),
-// whose staged diagonal and four epilogue inputs do not fit: held to 128 it
-// spilled 16 VGPRs to scratch.
-template <typename T, int ST, int EP>
+//
+// Grid transfers inside the kernel: as passes of their own they moved three more
+// vectors, and the launches around them one more each, at 4.2-4.6 of the 4.85
+// TB/s that a large copy reaches.  64^3, 16 cells in FP32: pre-smoothing 297 us
+// and restriction 92 us became one launch of 282 us, prolongation 106 us and
+// post-smoothing 227 us one of 285 us; these launches now keep the VALU 68% busy
+// (62% without a transfer), and that, not the vectors, is what bounds them.
+//  * RS (EP_PRE): the residual goes to the coarse right-hand side and never to
+//    memory.  The tile computes one more node row and column at its low j and
+//    k sides (and its chunk one more plane), so that every coarse node above
+//    its owned nodes has the 27 residuals of its full weighting in the
+//    workgroup; they pass through rb in LDS, plane by plane, and each coarse
+//    node's sum is carried in FP64 by one thread.
+//  * ST_PROLONG / ST_DPROLONG: the staged value is x + P xc, x read (PROLONG)
+//    or formed as b / (theta D) (DPROLONG: the degree-1 pre-smoothing, whose x
+//    is then never stored).  The coarse nodes around the tile are staged into
+//    cl one coarse plane at a time, two slabs ahead; each staging slot keeps
+//    its interpolated value of the lower coarse plane.
+// Waves per SIMD the FP32 variants are compiled for: 4 (at most 128 VGPRs).
+template <typename T>
 constexpr int tiled_waves() {
-  return sizeof(T) == 4 ? ((ST == ST_DSCALE && EP == EP_STEP) ? 3 : 4) : kWaves64;
+  return sizeof(T) == 4 ? 4 : kWaves64;
 }
 
-template <typename T, int ST, int EP, int TJ, int TK>
-__global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(Dims g, const T *__restrict__ E,
+template <typename T, int ST, int EP, int TJ, int TK, bool RS>
+__global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, const T *__restrict__ E,
                                                                            ModeC<T> mc, OpArgs<T> a, int TI,
                                                                            int tiles_k, int tiles, int chunks) {
   constexpr int NT = TJ * TK;                           // threads = owned nodes per plane
-  constexpr int NJ = TJ + 2, NK = TK + 2, NS = NJ * NK;  // staged nodes (one-node halo)
-  constexpr int EJ = TJ + 1, EK = TK + 1, NE = EJ * EK;  // voxels touching the tile
+  constexpr int H = RS ? 1 : 0;                         // extra node row / column / plane at the low sides
+  constexpr int NJ = TJ + 2 + H, NK = TK + 2 + H, NS = NJ * NK;  // staged nodes (one-node halo)
+  constexpr int EJ = TJ + 1 + H, EK = TK + 1 + H, NE = EJ * EK;  // voxels touching the tile
   constexpr int QS = (NS + NT - 1) / NT, QE = (NE + NT - 1) / NT;
   static_assert(NT % 64 == 0 && QS <= 2 && QE <= 2, "tile shape");
+  constexpr bool kProl = ST == ST_PROLONG || ST == ST_DPROLONG;
+  constexpr bool kStD = ST == ST_DSCALE || ST == ST_DPROLONG;  // stages b / (theta D)
+  constexpr int CJ = TJ / 2 + 2, CK = TK / 2 + 2;              // coarse nodes around the tile (kProl)
   constexpr unsigned SZ = sizeof(T);
   const int L = xcd_order(blockIdx.x, gridDim.x);
   const int lc = L % kRHS, tile = (L / kRHS) % tiles, chunk = (L / (kRHS * tiles)) % chunks;
@@ -305,6 +337,8 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
   const T bt = ST == ST_PUPD ? (T)a.beta[r] : (T)0;
   __shared__ T up[2][3 * NS];
   __shared__ T eo[NE * kEOH];
+  __shared__ T cl[kProl ? 3 * CJ * CK : 1];
+  __shared__ T rb[RS ? 3 * (TJ + 1) * (TK + 1) : 1];
   const int tid = threadIdx.x;
   // staging slots and voxels go to threads in an order rotated by a wave per
   // workgroup, so that the second round of the extra ones does not fall on
@@ -317,8 +351,7 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
   const int plane = g.ny * g.nz;
 
   // per-thread staging slots (fixed across planes): node offsets in a plane
-  int soff[QS], sjc[QS][2], skc[QS][2];
-  float sjw[QS], skw[QS];
+  int soff[QS];
 #pragma unroll
   for (int q = 0; q < QS; q++) {
     const int t = vt + q * NT;
@@ -326,16 +359,8 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
     if (t < NS) {
       const int nj = t / NK, nk = t - nj * NK;
       // slots of a tile wider than the grid wrap more than once
-      const int jj = ((j0 - 1 + nj) % g.ny + g.ny) % g.ny, kk = ((k0 - 1 + nk) % g.nz + g.nz) % g.nz;
+      const int jj = ((j0 - 1 - H + nj) % g.ny + g.ny) % g.ny, kk = ((k0 - 1 - H + nk) % g.nz + g.nz) % g.nz;
       soff[q] = jj * g.nz + kk;
-      if (ST == ST_PROLONG) {
-        sjc[q][0] = jj >> 1;
-        sjc[q][1] = ((jj + 1) >> 1) % a.gc.ny;
-        sjw[q] = (jj & 1) ? 0.5f : 1.0f;
-        skc[q][0] = kk >> 1;
-        skc[q][1] = ((kk + 1) >> 1) % a.gc.nz;
-        skw[q] = (kk & 1) ? 0.5f : 1.0f;
-      }
     }
   }
   // per-thread voxels (fixed across slabs): modulus offsets in a plane
@@ -346,15 +371,70 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
     eoff[q] = -1;
     if (e < NE) {
       const int ej = e / EK, ek = e - ej * EK;
-      const int jj = ((j0 - 1 + ej) % g.ny + g.ny) % g.ny, kk = ((k0 - 1 + ek) % g.nz + g.nz) % g.nz;
+      const int jj = ((j0 - 1 - H + ej) % g.ny + g.ny) % g.ny, kk = ((k0 - 1 - H + ek) % g.nz + g.nz) % g.nz;
       eoff[q] = jj * g.nz + kk;
     }
   }
 
-  // staging of node plane ip into LDS buffer buf.  PLAIN / DSCALE / PUPD are
-  // software-pipelined: fetch() issues the loads of a plane into registers
-  // one slab ahead, put() scales and stores them.  PROLONG (one sample only)
-  // stages directly.
+  // Coarse nodes of the fused prolongation: thread t < CJ CK brings node
+  // (j0/2 - 1 + t / CK, k0/2 - 1 + t % CK) of a coarse plane from memory (cfetch,
+  // two slabs ahead) to cl (cput).  A slot's 2D value (interp) adds two rows of
+  // two columns with weights (1, 0) at even and (1/2, 1/2) at odd fine nodes.
+  // (the interpolated value of the lower coarse plane: a thread's first slot
+  // keeps it in registers, the second slots in LDS, as with the voxels below)
+  constexpr int NSX = NS > NT ? NS - NT : 1;
+  __shared__ T ic[kProl ? 3 * NSX : 1];
+  T cr[3], ia[3];
+  unsigned coff = 0;
+  __amdgpu_buffer_rsrc_t rC = rU;
+  unsigned CB = 0;
+  if constexpr (kProl) {
+    CB = (unsigned)a.gc.V * SZ;
+    rC = brsrc(a.xc + (size_t)r * 3 * a.gc.V, 3 * CB);
+    const int cj = ((j0 / 2 - 1 + tid / CK) % a.gc.ny + a.gc.ny) % a.gc.ny,
+              ck = ((k0 / 2 - 1 + tid % CK) % a.gc.nz + a.gc.nz) % a.gc.nz;
+    coff = (unsigned)(cj * a.gc.nz + ck);
+  }
+  auto cfetch = [&](int I) {
+    if (tid < CJ * CK) {
+      const unsigned vo = ((unsigned)(wrap1(I, a.gc.nx) * a.gc.ny * a.gc.nz) + coff) * SZ;
+#pragma unroll
+      for (int c = 0; c < 3; c++) cr[c] = bload(rC, vo, c * CB, (T *)nullptr);
+    }
+  };
+  auto cput = [&]() {
+    if (tid < CJ * CK) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) cl[3 * tid + c] = cr[c];
+    }
+  };
+  // slot (nj, nk) is fine node (j0 - 1 + nj, k0 - 1 + nk): odd where nj is even.
+  // Its place in cl and its parities are packed in one register, which passes
+  // through an empty asm so that what derives from it is formed where it is
+  // used instead of being kept in seven registers over the loop.
+  int cpk[QS];
+#pragma unroll
+  for (int q = 0; q < QS; q++) {
+    const int t = vt + q * NT, nj = t / NK, nk = t - nj * NK;
+    cpk[q] = (3 * (((nj + 1) >> 1) * CK + ((nk + 1) >> 1))) << 2 | (nj & 1) << 1 | (nk & 1);
+  }
+  auto interp = [&](int q, T (&v)[3]) {
+    int pk = cpk[q];
+    asm volatile("" : "+v"(pk));
+    const T *row0 = cl + (pk >> 2);
+    const int dj = (pk & 2) ? 0 : 3 * CK, dk = (pk & 1) ? 0 : 3;
+    const T wj0 = (pk & 2) ? (T)1 : (T)0.5, wj1 = (pk & 2) ? (T)0 : (T)0.5;
+    const T wk0 = (pk & 1) ? (T)1 : (T)0.5, wk1 = (pk & 1) ? (T)0 : (T)0.5;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const T s0 = wk0 * row0[c] + wk1 * row0[dk + c], s1 = wk0 * row0[dj + c] + wk1 * row0[dj + dk + c];
+      v[c] = wj0 * s0 + wj1 * s1;
+    }
+  };
+
+  // staging of node plane ip into LDS buffer buf, software-pipelined: fetch()
+  // issues the loads of a plane into registers one slab ahead, put() scales
+  // and stores them.
   T pf[QS][3], pd[QS][3];
   auto fetch = [&](int ip) {
     const int iw = wrap1(ip, g.nx);
@@ -365,60 +445,82 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
 #pragma unroll
       for (int c = 0; c < 3; c++) {
         pf[q][c] = bload(rU, vo, c * VB, (T *)nullptr);
-        if (ST == ST_DSCALE) pd[q][c] = bload(rD, vo, c * VB, (T *)nullptr);
+        if (kStD) pd[q][c] = bload(rD, vo, c * VB, (T *)nullptr);
         if (ST == ST_PUPD) pd[q][c] = bload(rU2, vo, c * VB, (T *)nullptr);
       }
     }
   };
-  auto put = [&](int buf) {
+  auto put = [&](int buf, int ip) {
 #pragma unroll
     for (int q = 0; q < QS; q++) {
       if (soff[q] < 0) continue;
       T *dst = &up[buf][3 * (vt + q * NT)];
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        dst[c] = (ST == ST_DSCALE) ? pf[q][c] * (ti * pd[q][c])
-                 : (ST == ST_PUPD) ? pf[q][c] + bt * pd[q][c]
-                                   : pf[q][c];
-    }
-  };
-  auto stage = [&](int buf, int ip) {
-    if (ST != ST_PROLONG) {
-      fetch(ip);
-      put(buf);
-      return;
-    }
-    const int iw = wrap1(ip, g.nx);
-#pragma unroll
-    for (int q = 0; q < QS; q++) {
-      if (soff[q] < 0) continue;
-      const int t = vt + q * NT;
-      const int n = iw * plane + soff[q];
       T v[3];
 #pragma unroll
-      for (int c = 0; c < 3; c++) v[c] = a.u[off + (size_t)c * V + n];
-      const int ci0 = iw >> 1, ci1 = ((iw + 1) >> 1) % a.gc.nx;
-      const float wi = (iw & 1) ? 0.5f : 1.0f;
-      const int ni = (iw & 1) ? 2 : 1, nj = (sjw[q] < 1.0f) ? 2 : 1, nk = (skw[q] < 1.0f) ? 2 : 1;
-      const T w = (T)(wi * sjw[q] * skw[q]);
-      const size_t offc = (size_t)r * 3 * a.gc.V;
-      T sum[3] = {0, 0, 0};
-      for (int ai = 0; ai < ni; ai++)
-        for (int aj = 0; aj < nj; aj++)
-          for (int ak = 0; ak < nk; ak++) {
-            const int N = ((ai ? ci1 : ci0) * a.gc.ny + sjc[q][aj]) * a.gc.nz + skc[q][ak];
+      for (int c = 0; c < 3; c++)
+        v[c] = kStD ? pf[q][c] * (ti * pd[q][c]) : (ST == ST_PUPD) ? pf[q][c] + bt * pd[q][c] : pf[q][c];
+      if constexpr (kProl) {
+        // (x is rounded before the correction is added, as when it is stored)
+#pragma clang fp contract(off)
+        T *ix = ic + (vt + q * NT - NT);  // (second slots only)
+        if (ip & 1) {
+          T ib[3];
+          interp(q, ib);
 #pragma unroll
-            for (int c = 0; c < 3; c++) sum[c] += a.xc[offc + (size_t)c * a.gc.V + N];
+          for (int c = 0; c < 3; c++) {
+            v[c] = v[c] + (T)0.5 * ((q == 0 ? ia[c] : ix[c * NSX]) + ib[c]);
+            if (q == 0)
+              ia[c] = ib[c];
+            else
+              ix[c * NSX] = ib[c];
           }
+        } else {
 #pragma unroll
-      for (int c = 0; c < 3; c++) up[buf][3 * t + c] = v[c] + w * sum[c];
+          for (int c = 0; c < 3; c++) v[c] = v[c] + (q == 0 ? ia[c] : ix[c * NSX]);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++) dst[c] = v[c];
     }
   };
 
   const int nj = tid / TK, nk = tid % TK;  // owned node, output tile coords
   const int gj = j0 + nj, gk = k0 + nk;
   const bool owns = (gj < g.ny) && (gk < g.nz);
-  const int ot = 3 * ((nj + 1) * NK + nk + 1);  // owned node in the staged plane
+  const int ot = 3 * ((nj + 1 + H) * NK + nk + 1 + H);  // owned node in the staged plane
+  // RS: the extra nodes, row j0 - 1 (k0 - 1 ..) and column k0 - 1 (j0 ..)
+  const int xa = tid <= TK ? 0 : tid - TK, xb = tid <= TK ? tid : 0;
+  const bool extra = RS && tid < TJ + TK + 1;
+  unsigned xoff = 0;
+  if constexpr (RS) {
+    const int jj = ((j0 - 1 + xa) % g.ny + g.ny) % g.ny, kk = ((k0 - 1 + xb) % g.nz + g.nz) % g.nz;
+    xoff = (unsigned)(jj * g.nz + kk);
+  }
+  const __amdgpu_buffer_rsrc_t rB = brsrc(RS ? a.b + off : a.u + off, 3 * VB);
+  double racc = 0;  // RS: this thread's coarse node sum
+  // RS: restriction of residual plane ip in rb: rows and columns with weights
+  // 1/2, 1, 1/2, planes 2I - 1, 2I, 2I + 1 into coarse plane I
+  auto restrict_plane = [&](int ip) {
+    constexpr int CN = (TJ / 2) * (TK / 2);
+    if (tid >= 3 * CN) return;
+    const int c = tid / CN, q = tid - c * CN, J = q / (TK / 2), K = q - J * (TK / 2);
+    const T *p = rb + c * (TJ + 1) * (TK + 1) + 2 * J * (TK + 1) + 2 * K;
+    double s = 0;
+#pragma unroll
+    for (int oj = 0; oj < 3; oj++) {
+      const T *row = p + oj * (TK + 1);
+      const double rs = 0.5 * (double)row[0] + (double)row[1] + 0.5 * (double)row[2];
+      s += (oj == 1 ? 1.0 : 0.5) * rs;
+    }
+    if (ip & 1) {
+      const int I = (ip - 1) >> 1, gJ = j0 / 2 + J, gK = k0 / 2 + K;
+      if (ip > i0 && gJ < a.gc.ny && gK < a.gc.nz)
+        a.y[((size_t)r * 3 + c) * a.gc.V + ((size_t)I * a.gc.ny + gJ) * a.gc.nz + gK] = (T)(racc + 0.5 * s);
+      racc = 0.5 * s;
+    } else {
+      racc = racc + s;
+    }
+  };
   DotAcc dv;
 
   // Per voxel (three components, corners v = 4 bi + 2 bj + bk) the cube-mode
@@ -430,8 +532,13 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
   // face; the top face of slab s-1 and the bottom face of slab s lie on the
   // same node plane s, so they are summed before one inverse face transform
   // -- plane s is then complete after a single LDS exchange.
+  // A thread's first voxel keeps these values in registers; the few second
+  // ones (NE - NT of the tile) keep theirs in LDS, where only their own thread
+  // touches them: in registers they would cost every thread 24.
   constexpr bool kReuse = sizeof(T) == 4;
-  T ftop[QE][3][4], tmod[QE][3][4];
+  constexpr int NX = NE > NT ? NE - NT : 1;
+  __shared__ T carry[(kReuse ? 24 : 12) * NX];
+  T ftop[3][4], tmod[3][4];
   auto face_load = [&](int buf, int ej, int ek, T (&f)[3][4]) {
     const T *src = &up[buf][3 * (ej * NK + ek)];
 #pragma unroll
@@ -468,9 +575,35 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
           }
   };
 
-  stage(0, i0 - 1);
-  if (ST != ST_PROLONG) fetch(i0);
-  for (int sl = i0 - 1, p = 0; sl < iend; sl++, p++) {
+  if constexpr (kProl) {
+    // (i0 is even: the first staged plane, i0 - 1, lies between coarse planes
+    // i0/2 - 1 and i0/2)
+    cfetch(i0 / 2 - 1);
+    cput();
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < QS; q++) {
+      if (soff[q] < 0) continue;
+      T v[3];
+      interp(q, v);
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        if (q == 0)
+          ia[c] = v[c];
+        else
+          ic[c * NSX + vt + q * NT - NT] = v[c];
+      }
+    }
+    cfetch(i0 / 2);
+    __syncthreads();
+    cput();
+    cfetch(i0 / 2 + 1);
+    __syncthreads();
+  }
+  fetch(i0 - 1 - H);
+  put(0, i0 - 1 - H);
+  fetch(i0 - H);
+  for (int sl = i0 - 1 - H, p = 0; sl < iend; sl++, p++) {
     const int cur = p & 1, nxt = cur ^ 1;
     const int sw = wrap1(sl, g.nx);
     // loads in the order they are consumed: moduli of this slab, epilogue
@@ -479,20 +612,34 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
 #pragma unroll
     for (int q = 0; q < QE; q++)
       Ev[q] = eoff[q] >= 0 ? bload(rE, (unsigned)(sw * plane + eoff[q]) * SZ, 0u, (T *)nullptr) : (T)0;
-    const size_t nown = (size_t)sl * plane + gj * g.nz + gk;
+    const size_t nown = (size_t)sw * plane + gj * g.nz + gk;
     EpiIn<T> pin;
-    if ((EP != EP_AX || a.ydinv) && sl >= i0 && owns) epi_load<T, EP>(a, Ds, off, V, (int)nown, pin);
-    if (ST != ST_PROLONG) {
-      put(nxt);
-      if (sl + 2 <= iend) fetch(sl + 2);
-    } else {
-      stage(nxt, sl + 1);
+    if (EP != EP_AX && p > 0 && owns) epi_load<T, ST, EP>(a, Ds, off, V, (int)nown, pin);
+    T xin[3];
+    if constexpr (RS) {
+      if (p > 0 && extra) {
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+          xin[c] = bload(rB, ((unsigned)(sw * plane) + xoff) * SZ, c * VB, (T *)nullptr);
+      }
     }
+    put(nxt, sl + 1);
+    if (sl + 2 <= iend) fetch(sl + 2);
     // (this buffer was last read before the barrier that closed the previous
     // slab; the previous slab's gather of eo is behind that barrier too)
     __syncthreads();
+    if constexpr (RS) {
+      if (p > 1) restrict_plane(sl - 1);
+    }
+    if constexpr (kProl) {
+      // (the odd plane that reads cl is put in the next slab)
+      if (!(p & 1)) {
+        cput();
+        cfetch((sl + 1) / 2 + 2);
+      }
+    }
     T uo[3];
-    if (p > 0 && sl >= i0 && owns) {
+    if (EP != EP_PRE && p > 0 && owns) {
 #pragma unroll
       for (int c = 0; c < 3; c++) uo[c] = up[cur][ot + c];
     }
@@ -504,11 +651,12 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
       T fb[3][4], ft[3][4];
       face_load(nxt, ej, ek, ft);
       face_fwd(ft);
+      T *cy = carry + (e - NT);  // (second voxels only)
       if (kReuse && p > 0) {
 #pragma unroll
         for (int c = 0; c < 3; c++)
 #pragma unroll
-          for (int v = 0; v < 4; v++) fb[c][v] = ftop[q][c][v];
+          for (int v = 0; v < 4; v++) fb[c][v] = q == 0 ? ftop[c][v] : cy[(12 + 4 * c + v) * NX];
       } else {
         face_load(cur, ej, ek, fb);
         face_fwd(fb);
@@ -517,7 +665,12 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
 #pragma unroll
         for (int c = 0; c < 3; c++)
 #pragma unroll
-          for (int v = 0; v < 4; v++) ftop[q][c][v] = ft[c][v];
+          for (int v = 0; v < 4; v++) {
+            if (q == 0)
+              ftop[c][v] = ft[c][v];
+            else
+              cy[(12 + 4 * c + v) * NX] = ft[c][v];
+          }
       }
       // i stage: modes sm = 4 si + s_jk
       T w[3][8];
@@ -532,9 +685,13 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
       // (plane sl+1) modal forces.  FP64 folds the two per component (fewer
       // live registers); FP32 keeps them apart, which schedules without
       // spills at 4 waves per SIMD
-      T bm[3][4];
+      T bm[3][4], tm[3][4];
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) tm[c][v] = q == 0 ? tmod[c][v] : cy[(4 * c + v) * NX];
       if constexpr (sizeof(T) == 8) {
-        couple_split<T>(w, Ev[q], mc, bm, tmod[q], p > 0);
+        couple_split<T>(w, Ev[q], mc, bm, tm, p > 0);
       } else {
         T z[3][8];
         mode_couple<T>(w, Ev[q], mc, z);
@@ -543,10 +700,19 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
 #pragma unroll
           for (int v = 0; v < 4; v++) {
             bm[c][v] = z[c][v] - z[c][4 + v];
-            if (p > 0) bm[c][v] += tmod[q][c][v];
-            tmod[q][c][v] = z[c][v] + z[c][4 + v];
+            if (p > 0) bm[c][v] += tm[c][v];
+            tm[c][v] = z[c][v] + z[c][4 + v];
           }
       }
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          if (q == 0)
+            tmod[c][v] = tm[c][v];
+          else
+            cy[(4 * c + v) * NX] = tm[c][v];
+        }
       if (p > 0) {
         face_inv(bm);
         T *dst = eo + e * kEOH;
@@ -556,30 +722,52 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
           for (int c = 0; c < 3; c++) dst[3 * v + c] = bm[c][v];
       }
     }
-    // plane i0 - 1 is not owned (uniform branch); its buffer is read above
+    // the first slab completes no plane (uniform branch); its buffer is read above
     // and refilled by the next slab's put, so the slab still closes with a
     // barrier
     __syncthreads();
     if (p == 0) continue;
-    // plane sl: voxel columns (nj+dj, nk+dk) hold this node as face corner
+    // plane sl: voxel columns (a+dj, b+dk) hold this node as face corner
     // (1-dj, 1-dk)
-    if (sl >= i0 && owns) {
-      T Au[3] = {0, 0, 0};
+    auto gather = [&](int na, int nb, T (&Au)[3]) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) Au[c] = 0;
 #pragma unroll
       for (int dj = 0; dj < 2; dj++)
 #pragma unroll
         for (int dk = 0; dk < 2; dk++) {
-          const T *src = eo + ((nj + dj) * EK + nk + dk) * kEOH + 3 * (2 * (1 - dj) + (1 - dk));
+          const T *src = eo + ((na + dj) * EK + nb + dk) * kEOH + 3 * (2 * (1 - dj) + (1 - dk));
 #pragma unroll
           for (int c = 0; c < 3; c++) Au[c] += src[c];
         }
+    };
+    if constexpr (RS) {
+      T Au[3];
+      if (owns) {
+        gather(nj + 1, nk + 1, Au);
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+          rb[(c * (TJ + 1) + nj + 1) * (TK + 1) + nk + 1] = pin.e0[c] - Au[c];
+      }
+      if (extra) {
+        gather(xa, xb, Au);
+#pragma unroll
+        for (int c = 0; c < 3; c++) rb[(c * (TJ + 1) + xa) * (TK + 1) + xb] = xin[c] - Au[c];
+      }
+    } else if (owns) {
+      T Au[3];
+      gather(nj, nk, Au);
       if (a.nt)  // (one uniform branch per node, not per store)
-        epilogue<T, EP, true>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
+        epilogue<T, ST, EP, true>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
       else
-        epilogue<T, EP, false>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
+        epilogue<T, ST, EP, false>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
     }
   }
-  if ((EP == EP_AX || EP == EP_STEP || EP == EP_RES || EP == EP_CHEB0) && a.dot) {
+  if constexpr (RS) {
+    __syncthreads();
+    restrict_plane(iend - 1);
+  }
+  if ((EP == EP_AX || EP == EP_RES || EP == EP_FIN1 || EP == EP_LASTD) && a.dot) {
     const int pidx = chunk * tiles + tile;
     block_partial(a.red, a.slot, r, pidx, block_sum_n<NT>(dv.a));
     if (EP == EP_RES) {
@@ -595,7 +783,7 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, EP>())) void k_tiled(D
 template <typename T, int TJ, int TK>
 static int tiled_resident_of() {
   int per_cu = 0, dev = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiled<T, ST_PLAIN, EP_STEP, TJ, TK>, TJ * TK, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_tiled<T, ST_PLAIN, EP_STEP, TJ, TK, false>, TJ * TK, 0) !=
           hipSuccess ||
       hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu < 1 ||
@@ -623,7 +811,8 @@ template <typename T, int ST, int EP, int TJ, int TK>
 static void tiled_go(const Dims &g, int R, const T *E, const ModeC<T> &mc, const OpArgs<T> &a,
                      hipStream_t s, int shape, hipEvent_t ev0, hipEvent_t ev1) {
   const int tiles_k = (g.nz + TK - 1) / TK, tiles_j = (g.ny + TJ - 1) / TJ;
-  const int TI = tiled_chunk(g, R, shape, (int)sizeof(T));
+  constexpr bool fused = EP == EP_PRE || ST == ST_PROLONG || ST == ST_DPROLONG;
+  const int TI = tiled_chunk(g, R, shape, (int)sizeof(T), fused);
   const int tiles = tiles_j * tiles_k, chunks = (g.nx + TI - 1) / TI;
   // non-temporal output stores once one output vector (all right-hand
   // sides) passes 128 MiB: 64^3 x 16 cells (302 MB in FP32) gains 1-2% from
@@ -633,16 +822,19 @@ static void tiled_go(const Dims &g, int R, const T *E, const ModeC<T> &mc, const
   OpArgs<T> an = a;
   an.nt = (size_t)R * 3 * (size_t)g.V * sizeof(T) >= ((size_t)128 << 20) ? 1 : 0;
   if (R % kRHS) throw std::runtime_error("right-hand sides must come in groups of six");
+  if (fused &&
+      (a.gc.nx * 2 != g.nx || a.gc.ny * 2 != g.ny || a.gc.nz * 2 != g.nz || (TI & 1)))
+    throw std::runtime_error("fused grid transfers need the halved grid and chunks of even length");
   // buffer resources address a right-hand side's vector with 32-bit offsets
   if ((size_t)3 * g.V * sizeof(T) >= ((size_t)1 << 31)) throw std::runtime_error("grid too large for the tiled operator");
   if (ev0) {
     // timed launch: the runtime records the events at the kernel's own start
     // and end, so no queue gap is counted
-    hipExtLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, ev0, ev1,
+    hipExtLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, ev0, ev1,
                           0, g, E, mc, an, TI, tiles_k, tiles, chunks);
     return;
   }
-  hipLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, g, E, mc, an,
+  hipLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, g, E, mc, an,
                      TI, tiles_k, tiles, chunks);
 }
 
@@ -688,13 +880,20 @@ void launch_tiled(int st, int ep, const Dims &g, int R, const T *E, const ModeCo
     return;                                            \
   }
   GO(ST_PLAIN, EP_AX)
+  GO(ST_PLAIN, EP_AXD)
   GO(ST_PUPD, EP_AX)
   GO(ST_PLAIN, EP_RES)
+  GO(ST_PLAIN, EP_PRE)
+  GO(ST_DSCALE, EP_PRE)
   GO(ST_DSCALE, EP_STEP)
+  GO(ST_DSCALE, EP_LAST)
   GO(ST_PLAIN, EP_STEP)
+  GO(ST_PLAIN, EP_LAST)
+  GO(ST_PLAIN, EP_LASTD)
   GO(ST_PROLONG, EP_CHEB0)
-  GO(ST_PLAIN, EP_CHEB0)
-  GO(ST_DSCALE, EP_CHEB0)
+  GO(ST_PROLONG, EP_FIN1)
+  GO(ST_DPROLONG, EP_CHEB0)
+  GO(ST_DPROLONG, EP_FIN1)
 #undef GO
   throw std::runtime_error("no operator kernel for this stage/epilogue pair");
 }
@@ -776,8 +975,8 @@ __device__ __forceinline__ void stencil_node(const Dims &g, const T *__restrict_
     for (int c = 0; c < 3; c++) uo[c] = stage_at<T, ST>(a, Ds, ti, off, V, c, n);
     DotAcc dv;
     EpiIn<T> pin;
-    epi_load<T, EP>(a, Ds, off, V, n, pin);
-    epilogue<T, EP>(a, pin, ti, c1, c2, off, V, n, acc[t], uo, dv);
+    epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
+    epilogue<T, ST, EP>(a, pin, ti, c1, c2, off, V, n, acc[t], uo, dv);
   }
 }
 
@@ -856,8 +1055,8 @@ __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims
   const T c1 = a.cheb ? (T)a.cheb[kMaxB + smp] : (T)0, c2 = a.cheb ? (T)a.cheb[2 * kMaxB + smp] : (T)0;
   DotAcc dv;
   EpiIn<T> pin;
-  epi_load<T, EP>(a, Ds, off, V, n, pin);
-  epilogue<T, EP>(a, pin, ti, c1, c2, off, V, n, Au, uo, dv);
+  epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
+  epilogue<T, ST, EP>(a, pin, ti, c1, c2, off, V, n, Au, uo, dv);
 }
 
 // One-plane form of the tiled stencil kernel, for levels with planes of at
@@ -1032,8 +1231,8 @@ __global__ __launch_bounds__(kBlock) void k_stencil_plane(Dims g, const T *__res
       const size_t off = off0 + (size_t)t * 3 * V;
       DotAcc dv;
       EpiIn<T> pin;
-      epi_load<T, EP>(a, Ds, off, V, n, pin);
-      epilogue<T, EP>(a, pin, ti, c1, c2, off, V, n, acc[t], uo[t], dv);
+      epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
+      epilogue<T, ST, EP>(a, pin, ti, c1, c2, off, V, n, acc[t], uo[t], dv);
     }
   }
 }
@@ -1074,11 +1273,15 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
     return;                                                                                      \
   }
   GO(ST_PLAIN, EP_AX)
-  GO(ST_PLAIN, EP_RES)
+  GO(ST_PLAIN, EP_AXD)
+  GO(ST_PLAIN, EP_PRE)
+  GO(ST_DSCALE, EP_CHEB0L)
   GO(ST_DSCALE, EP_STEP)
+  GO(ST_DSCALE, EP_LAST)
   GO(ST_PLAIN, EP_STEP)
+  GO(ST_PLAIN, EP_LAST)
   GO(ST_PLAIN, EP_CHEB0)
-  GO(ST_DSCALE, EP_CHEB0)
+  GO(ST_PLAIN, EP_FIN1)
 #undef GO
   throw std::runtime_error("no operator kernel for this stage/epilogue pair");
 }

@@ -222,20 +222,19 @@ double tiled_alg_bytes(int st, int ep, const OpArgs<T> &a, double V, double sz, 
     in[nin++] = p;
   };
   if (st == ST_PUPD) add_in(a.u2);
-  if (ep == EP_RES || ep == EP_CHEB0) add_in(a.b);
-  if (ep == EP_STEP) {
+  const bool step = ep == EP_STEP || ep == EP_LAST || ep == EP_LASTD;
+  if (ep == EP_RES || ep == EP_PRE || ep == EP_CHEB0 || ep == EP_FIN1 || ep == EP_LASTD) add_in(a.b);
+  if (step) {
     add_in(a.rprev);
-    add_in(a.xprev);
-    if (a.dot) add_in(a.b);
+    if (st != ST_DSCALE) add_in(a.xprev);
   }
-  double vec_out = 0;
-  if (ep == EP_AX) vec_out = 1 + (a.pout ? 1 : 0);
-  if (ep == EP_RES) vec_out = 1;
-  if (ep == EP_CHEB0) vec_out = a.fin1 ? 1 : (a.last ? 2 : 3);
-  if (ep == EP_STEP) vec_out = a.last ? 1 : 3;
-  double vec = nin + vec_out;
-  if (st == ST_PROLONG) vec += 0.125;  // coarse correction, 1/8 of the nodes
-  const bool usesD = st == ST_DSCALE || ep == EP_CHEB0 || ep == EP_STEP || (ep == EP_AX && a.ydinv);
+  double vec = nin;
+  if (ep == EP_AX) vec += st == ST_PUPD ? 2 : 1;
+  if (ep == EP_AXD || ep == EP_RES || ep == EP_FIN1 || ep == EP_LAST || ep == EP_LASTD) vec += 1;
+  if (ep == EP_PRE) vec += 0.125;  // the restricted residual
+  if (ep == EP_CHEB0 || ep == EP_STEP) vec += 3;
+  if (st == ST_PROLONG || st == ST_DPROLONG) vec += 0.125;  // coarse correction, 1/8 of the nodes
+  const bool usesD = st == ST_DSCALE || st == ST_DPROLONG || ep == EP_CHEB0 || ep == EP_FIN1 || step || ep == EP_AXD;
   return V * (3.0 * sz * Rn * vec + ns * sz * (usesD ? 4.0 : 1.0));
 }
 
@@ -246,13 +245,13 @@ void Context::op(Hierarchy<T> &h, int l, int st, int ep, OpArgs<T> a) {
   if (!a.Dinv) a.Dinv = L.Dinv.template as<T>();
   if (l == 0) {
     const Dims &g0 = L.g;
-    const bool dense = o.apply_kernel == 1 && st == ST_PLAIN && (ep == EP_AX || ep == EP_RES);
+    const bool dense = o.apply_kernel == 1 && st == ST_PLAIN && (ep == EP_AX || ep == EP_AXD || ep == EP_RES);
     auto launch = [&](hipEvent_t e0, hipEvent_t e1) {
       if (dense) {
         FineOp<T> f{g0, h.E.template as<T>(), h.Ke.template as<T>()};
         launch_dense_apply<T>(f, R, a.u, a.y, a.b, ep == EP_RES ? 1 : 0, a.act,
                               a.dot ? &a.red : nullptr, a.slot, stream);
-        if (a.ydinv) launch_scale_by_dinv_norm<T>(g0.V, R, a.y, a.Dinv, a.act, red, stream);
+        if (ep == EP_AXD) launch_scale_by_dinv_norm<T>(g0.V, R, a.y, a.Dinv, a.act, red, stream);
       } else {
         launch_tiled<T>(st, ep, g0, R, h.E.template as<T>(), modecoef, a, stream, shape_fine, e0, e1);
       }
@@ -335,7 +334,7 @@ void Context::apply(Hierarchy<T> &h, int l, const T *u, T *y, const T *bb, int m
     a.slot = slot;
     a.dot = 1;
   }
-  op<T>(h, l, ST_PLAIN, mode == 1 ? EP_RES : EP_AX, a);
+  op<T>(h, l, ST_PLAIN, mode == 0 ? EP_AX : l == 0 ? EP_RES : EP_PRE, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -411,8 +410,7 @@ void Context::estimate_lmax(Hierarchy<T> &h) {
       a.u = xv;
       a.y = yv;
       a.act = ap;
-      a.ydinv = 1;
-      op<T>(h, (int)l, ST_PLAIN, EP_AX, a);
+      op<T>(h, (int)l, ST_PLAIN, EP_AXD, a);
       std::swap(xv, yv);
     }
     launch_dot<T>(V, R, yv, yv, S_AUX, ap, red, stream);  // y_9
@@ -690,123 +688,101 @@ void Context::set_cheb(const Hierarchy<T> &h, int l, OpArgs<T> &a, int step, dou
   a.cheb = h.cheb.template as<double>() + (((size_t)l * h.cheb_steps + step) * 2 + kind) * 3 * kMaxB;
 }
 
-// k Chebyshev steps on level l from x = 0 (pre-smoothing, and the coarsest
-// solve when that level is too large for the dense inverse)
+// k >= 2 Chebyshev steps on level l from x = 0 (pre-smoothing, and the
+// coarsest solve when that level is too large for the dense inverse)
 template <typename T>
 void Context::cheb_run(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_, int k, double ratio) {
   Level<T> &L = h.lv[l];
-  if (k == 1) {
-    // x = b / (theta D) as one fused DSCALE pass with c1 = c2 = 0
-    OpArgs<T> a;
-    a.act = act_;
-    a.u = bb;
-    a.rprev = bb;
-    a.r = L.r.template as<T>();
-    a.x = xx;
-    a.dout = L.d.template as<T>();
-    a.last = 1;  // c1 = c2 = 0: x = staged value
-    set_cheb(h, l, a, 0, ratio);
-    op<T>(h, l, ST_DSCALE, EP_STEP, a);
-    return;
-  }
   T *dcur = L.d.template as<T>(), *dnxt = L.d2.template as<T>();
   OpArgs<T> a;
   a.act = act_;
   a.u = bb;
   a.rprev = bb;
-  a.xprev = nullptr;
+  a.xprev = xx;
   a.r = L.r.template as<T>();
   a.x = xx;
   a.dout = dcur;
-  a.last = (k == 2);
   set_cheb(h, l, a, 1, ratio);
-  op<T>(h, l, ST_DSCALE, EP_STEP, a);
+  op<T>(h, l, ST_DSCALE, k == 2 ? EP_LAST : EP_STEP, a);
+  a.rprev = L.r.template as<T>();
   for (int s = 2; s < k; s++) {
     a.u = dcur;
-    a.rprev = L.r.template as<T>();
-    a.xprev = xx;
     a.dout = dnxt;
-    a.last = (s == k - 1);
     set_cheb(h, l, a, s, ratio);
-    op<T>(h, l, ST_PLAIN, EP_STEP, a);
+    op<T>(h, l, ST_PLAIN, s == k - 1 ? EP_LAST : EP_STEP, a);
     std::swap(dcur, dnxt);
   }
 }
 
+// The fine level's pre-smoothing and restriction: C.b = P^T (b - A x) with x
+// the degree-nu1 smoothed iterate from zero, in L.xn (degree 1: x = b / (theta
+// D) is staged only, here and again in the post-smoothing, and never stored)
 template <typename T>
-void Context::pre_smooth(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_) {
-  cheb_run<T>(h, l, bb, xx, act_, nu_pre(l), o.cheby_ratio);
+void Context::pre_fine(Hierarchy<T> &h, const T *bb, const int *act_) {
+  Level<T> &L = h.lv[0];
+  Level<T> &C = h.lv[1];
+  OpArgs<T> a;
+  a.act = act_;
+  a.b = bb;
+  a.y = C.b.template as<T>();
+  a.gc = C.g;
+  if (o.nu1 == 1) {
+    a.u = bb;
+    set_cheb(h, 0, a, 0, o.cheby_ratio);
+    op<T>(h, 0, ST_DSCALE, EP_PRE, a);
+    return;
+  }
+  T *xn = L.xn.template as<T>();
+  cheb_run<T>(h, 0, bb, xn, act_, o.nu1, o.cheby_ratio);
+  a.u = xn;
+  op<T>(h, 0, ST_PLAIN, EP_PRE, a);
 }
 
-// Returns true when the last launch also left the partials of b . x in
-// dot_slot (fine level, degree >= 2).
+// The k = nu2 Chebyshev steps after the coarse correction x + P xc, on level l,
+// ending in xx.  The fine level stages the correction inside the first step;
+// the coarse levels add it in place first.  Returns true when the last launch
+// also left the partials of b . x in dot_slot (fine level).
 template <typename T>
 bool Context::post_smooth(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_, int dot_slot) {
   Level<T> &L = h.lv[l];
   Level<T> &C = h.lv[l + 1];
   const int k = nu_post(l);
+  const bool dot = l == 0 && dot_slot >= 0;
   OpArgs<T> a;
   a.act = act_;
   a.u = xx;
   a.b = bb;
   a.r = L.r.template as<T>();
   a.dout = L.d2.template as<T>();
-  a.x = L.xn.template as<T>();
+  a.x = xx;
+  a.red = red;
+  a.slot = dot_slot;
+  a.dot = dot;
   set_cheb(h, l, a, 0, o.cheby_ratio);
-  if (k == 1 && l == 0 && R > kRHS) {
-    // degree 1 at the fine level: xn = x + P xc out of place, then one launch
-    // leaves the smoothed x (and, fused, the partials of b . x = r . z)
-    launch_prolong_add<T>(L.g, C.g, R, C.x.template as<T>(), xx, act_, stream, L.xn.template as<T>(),
-                          xfer_shape(l));
-    a.u = L.xn.template as<T>();
-    a.x = xx;
-    a.fin1 = 1;
-    if (dot_slot >= 0) {
-      a.red = red;
-      a.slot = dot_slot;
-      a.dot = 1;
-    }
-    op<T>(h, l, ST_PLAIN, EP_CHEB0, a);
-    return dot_slot >= 0;
-  }
-  if (l == 0 && R <= kRHS) {
-    // one sample: staging x + P xc inside the operator saves a launch; with
-    // more right-hand sides the recomputed interpolation costs more than the
-    // separate pass
+  const int first = k == 1 ? EP_FIN1 : EP_CHEB0;
+  if (l == 0) {
+    a.u = o.nu1 == 1 ? bb : L.xn.template as<T>();
     a.xc = C.x.template as<T>();
     a.gc = C.g;
-    op<T>(h, l, ST_PROLONG, EP_CHEB0, a);  // x3 = x + P xc staged, kept in xn
+    op<T>(h, 0, o.nu1 == 1 ? ST_DPROLONG : ST_PROLONG, first, a);
   } else {
-    launch_prolong_add<T>(L.g, C.g, R, C.x.template as<T>(), xx, act_, stream, nullptr, xfer_shape(l));
-    op<T>(h, l, ST_PLAIN, EP_CHEB0, a);
-  }
-  if (k == 1) {
-    launch_add2<T>(L.g.V, R, L.xn.template as<T>(), L.d2.template as<T>(), xx, act_, stream);
-    return false;
+    // (out of place: the smoothing step stages xn and writes xx)
+    T *xn = L.xn.template as<T>();
+    launch_prolong_add<T>(L.g, C.g, R, C.x.template as<T>(), xx, act_, stream, xn, xfer_shape(l));
+    a.u = xn;
+    op<T>(h, l, ST_PLAIN, first, a);
   }
   T *dcur = L.d2.template as<T>(), *dnxt = L.d.template as<T>();
-  OpArgs<T> s1;
-  s1.act = act_;
-  s1.r = L.r.template as<T>();
-  s1.rprev = L.r.template as<T>();
-  s1.x = xx;
-  const bool fuse = l == 0 && dot_slot >= 0;
+  a.rprev = L.r.template as<T>();
+  a.xprev = xx;
   for (int s = 1; s < k; s++) {
-    s1.u = dcur;
-    s1.xprev = (s == 1) ? L.xn.template as<T>() : xx;
-    s1.dout = dnxt;
-    s1.last = (s == k - 1);
-    if (s1.last && fuse) {
-      s1.b = bb;
-      s1.red = red;
-      s1.slot = dot_slot;
-      s1.dot = 1;
-    }
-    set_cheb(h, l, s1, s, o.cheby_ratio);
-    op<T>(h, l, ST_PLAIN, EP_STEP, s1);
+    a.u = dcur;
+    a.dout = dnxt;
+    set_cheb(h, l, a, s, o.cheby_ratio);
+    op<T>(h, l, ST_PLAIN, s < k - 1 ? EP_STEP : dot ? EP_LASTD : EP_LAST, a);
     std::swap(dcur, dnxt);
   }
-  return fuse;
+  return dot;
 }
 
 template <typename T>
@@ -821,24 +797,26 @@ bool Context::vcycle(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_
   }
   Level<T> &L = h.lv[l];
   Level<T> &C = h.lv[l + 1];
-  if (nu_pre(l) == 1) {
-    // degree-1 pre-smoothing x = b / (theta D) needs no operator apply: one
-    // launch stages it and leaves the residual b - A x for the restriction
-    OpArgs<T> a;
-    a.act = act_;
-    a.u = bb;
-    a.b = bb;
-    a.r = L.r.template as<T>();
-    a.dout = L.d.template as<T>();
-    a.x = xx;
-    a.last = 1;
-    set_cheb(h, l, a, 0, o.cheby_ratio);
-    op<T>(h, l, ST_DSCALE, EP_CHEB0, a);
+  if (l == 0) {
+    pre_fine<T>(h, bb, act_);
   } else {
-    pre_smooth<T>(h, l, bb, xx, act_);
-    apply<T>(h, l, xx, L.r.template as<T>(), bb, 1, act_, nullptr, 0);
+    if (nu_pre(l) == 1) {
+      // degree-1 pre-smoothing x = b / (theta D) needs no operator apply: one
+      // launch stages it and leaves the residual b - A x for the restriction
+      OpArgs<T> a;
+      a.act = act_;
+      a.u = bb;
+      a.b = bb;
+      a.r = L.r.template as<T>();
+      a.x = xx;
+      set_cheb(h, l, a, 0, o.cheby_ratio);
+      op<T>(h, l, ST_DSCALE, EP_CHEB0L, a);
+    } else {
+      cheb_run<T>(h, l, bb, xx, act_, nu_pre(l), o.cheby_ratio);
+      apply<T>(h, l, xx, L.r.template as<T>(), bb, 1, act_, nullptr, 0);
+    }
+    launch_restrict<T>(L.g, C.g, R, L.r.template as<T>(), C.b.template as<T>(), act_, stream, xfer_shape(l));
   }
-  launch_restrict<T>(L.g, C.g, R, L.r.template as<T>(), C.b.template as<T>(), act_, stream, xfer_shape(l));
   vcycle<T>(h, l + 1, C.b.template as<T>(), C.x.template as<T>(), act_, -1);
   return post_smooth<T>(h, l, bb, xx, act_, dot_slot);
 }
@@ -859,15 +837,15 @@ void Context::precond(Hierarchy<T> &h, const T *rv, T *zv, const int *act_, int 
 }
 
 // the V-cycle's last fine-level smoothing launch also reduces r . z
-// (degree >= 2, or degree 1 on the multi-sample path)
 template <typename T>
 bool Context::fuses_rz(const Hierarchy<T> &h) const {
-  return o.precond == FEMH_PRECOND_MG && h.lv.size() > 1 && (o.nu2 >= 2 || (o.nu2 == 1 && R > kRHS));
+  return o.precond == FEMH_PRECOND_MG && h.lv.size() > 1;
 }
 
 template <typename T>
 int Context::rz_parts(const Hierarchy<T> &h) const {
-  return fuses_rz(h) ? tiled_parts(g, R, shape_fine, (int)sizeof(T)) : vec_parts(g.V);
+  // (degree 1: the launch that adds the coarse correction also ends the cycle)
+  return fuses_rz(h) ? tiled_parts(g, R, shape_fine, (int)sizeof(T), o.nu2 == 1) : vec_parts(g.V);
 }
 
 // PCG over all right-hand sides flagged in `active` (updated in place as

@@ -253,7 +253,7 @@ struct Context {
   void apply(Hierarchy<T> &h, int l, const T *u, T *y, const T *b, int mode, const int *act_,
              const Reduce *red, int slot);
   template <typename T>
-  void pre_smooth(Hierarchy<T> &h, int l, const T *b, T *x, const int *act_);
+  void pre_fine(Hierarchy<T> &h, const T *b, const int *act_);
   template <typename T>
   bool post_smooth(Hierarchy<T> &h, int l, const T *b, T *x, const int *act_, int dot_slot);
   template <typename T>
