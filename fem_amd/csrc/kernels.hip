@@ -947,6 +947,14 @@ __global__ __launch_bounds__(kBlock) void k_finalize(Reduce red, int slot, int n
   if (threadIdx.x == 0) red.scalars[slot * kSlotWidth + blockIdx.x] = s;
 }
 
+// partials [0, np_new) of (slot, RHS) = their sum over np_old, then zeros: a
+// reader that sums np_new of them gets the same value
+__global__ __launch_bounds__(kBlock) void k_collapse(Reduce red, int slot, int np_old, int np_new) {
+  const double s = sum_parts(red, slot, blockIdx.x, np_old);
+  double *pp = red.partials + ((size_t)slot * kSlotWidth + blockIdx.x) * kMaxPartials;
+  for (int i = threadIdx.x; i < np_new; i += kBlock) pp[i] = i == 0 ? s : 0.0;
+}
+
 __global__ void k_reduce_init(unsigned *ctr, double *scal, int n) {
   for (int t = threadIdx.x; t < n; t += blockDim.x) {
     ctr[t] = 0u;
@@ -1158,6 +1166,10 @@ int vec_parts(int V) { return grid_for(3 * V); }
 
 void launch_finalize(const Reduce &red, int slot, int nidx, int np, hipStream_t s) {
   hipLaunchKernelGGL(k_finalize, dim3(nidx), dim3(kBlock), 0, s, red, slot, np);
+}
+
+void launch_collapse(int R, int slot, const Reduce &red, int np_old, int np_new, hipStream_t s) {
+  hipLaunchKernelGGL(k_collapse, dim3(R), dim3(kBlock), 0, s, red, slot, np_old, np_new);
 }
 
 void reduce_init(Reduce &red, hipStream_t s) {

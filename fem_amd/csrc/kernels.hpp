@@ -89,6 +89,8 @@ struct StencilOp {
 int dense_parts(const Dims &g);  // partials written by a dense dot-apply
 int vec_parts(int V);             // partials of 3V-vector reductions
 void launch_finalize(const Reduce &red, int slot, int nidx, int np, hipStream_t s);
+// the np_old partials of every RHS as one partial followed by np_new - 1 zeros
+void launch_collapse(int R, int slot, const Reduce &red, int np_old, int np_new, hipStream_t s);
 
 // ---- fine level ---------------------------------------------------------
 // dense node-gather operator (diagnostic / cross-check of the tiled kernel):

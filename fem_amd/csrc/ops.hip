@@ -257,6 +257,35 @@ __device__ __forceinline__ int xcd_order(int b, int n) {
   return x * per + (x < rem ? x : rem) + slot;
 }
 
+// Work of a launch as (cell, unit, inner): `inner` workgroups share a unit's data
+// (load cases or their groups) and neighbouring units (tiles and planes of a
+// cell) share halos.  Two logical orders:
+//  * cell, unit, inner: neighbouring units follow each other on one XCD, but a
+//    cell lies on one or two XCDs, so the launches of a batch's last cells run
+//    there alone (48^3, one of 12 cells left: 65 us a fine launch of 324 active
+//    workgroups);
+//  * spread: eighth of the units, cell, unit within the eighth, inner: every
+//    XCD gets an eighth of every cell (that launch: 24 us).
+// Spread is taken for launches sized for a few remaining right-hand sides
+// (live_rhs), and whenever the units divide by eight, so that an eighth is a
+// block of whole neighbours and cells that converge early leave no XCD idle
+// (48 cells of 64^3: 77.1 -> 75.3 ms).  Elsewhere it costs more halo traffic
+// than it balances (40^3 in FP64, 18 units: 33.2 -> 39.3 ms).
+static inline int spread_rule(int sparse, int units) { return sparse || units % 8 == 0; }
+struct WorkId {
+  int cell, unit, inner;
+};
+__device__ __forceinline__ WorkId work_order(int b, int n, int cells, int units, int inner, int spread) {
+  const int L = xcd_order(b, n);
+  if (!spread) return {L / (inner * units), L / inner % units, L % inner};
+  const int q = L / (inner * cells);  // units before this workgroup's, all cells alike
+  int p = q * 8 / units;              // its eighth: units [p U / 8, (p + 1) U / 8)
+  while ((p + 1) * units / 8 <= q) p++;
+  const int u0 = p * units / 8, su = (p + 1) * units / 8 - u0;
+  const int rem = L - u0 * inner * cells, t = rem / inner;
+  return {t / su, u0 + t % su, rem - t * inner};
+}
+
 // raw buffer access: base pointer and byte range in a resource, one 32-bit
 // lane offset plus a scalar offset per access (no 64-bit address arithmetic)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t brsrc(const void *p, unsigned bytes) {
@@ -269,10 +298,9 @@ __device__ __forceinline__ double bload(__amdgpu_buffer_rsrc_t r, unsigned voff,
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
 
-// grid: one dimension of tiles * chunks * R workgroups; logical order (cell,
-// chunk, tile, load case), load case fastest, so that the six load cases of a
-// tile (same moduli and diagonal) and then the neighbouring tiles follow each
-// other on one XCD.
+// grid: one dimension of tiles * chunks * R workgroups, units of (chunk, tile)
+// with the six load cases of a tile (same moduli and diagonal) next to each
+// other on one XCD (work_order).
 //
 // LDS: staged node planes in a two-buffer ring, node-interleaved
 // (up[buf][3 * slot + c]), so that the 12 values of a voxel face and the
@@ -319,10 +347,9 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   constexpr bool kStD = ST == ST_DSCALE || ST == ST_DPROLONG;  // stages b / (theta D)
   constexpr int CJ = TJ / 2 + 2, CK = TK / 2 + 2;              // coarse nodes around the tile (kProl)
   constexpr unsigned SZ = sizeof(T);
-  const int L = xcd_order(blockIdx.x, gridDim.x);
-  const int lc = L % kRHS, tile = (L / kRHS) % tiles, chunk = (L / (kRHS * tiles)) % chunks;
-  const int smp = L / (kRHS * tiles * chunks);
-  const int r = smp * kRHS + lc;
+  const WorkId id = work_order(blockIdx.x, gridDim.x, gridDim.x / (kRHS * tiles * chunks), tiles * chunks, kRHS, a.spread);
+  const int smp = id.cell, tile = id.unit % tiles, chunk = id.unit / tiles;
+  const int r = smp * kRHS + id.inner;
   if (!a.act[r]) return;
   const int V = g.V;
   const unsigned VB = (unsigned)V * SZ;  // bytes per component plane
@@ -344,7 +371,7 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   // workgroup, so that the second round of the extra ones does not fall on
   // the same wave -- hence the same SIMD -- in every workgroup; owned nodes
   // (the epilogue) keep the plain thread order
-  const int vt = (tid + 64 * (L & (NT / 64 - 1))) & (NT - 1);
+  const int vt = (tid + 64 * ((int)(blockIdx.x >> 3) & (NT / 64 - 1))) & (NT - 1);
   const int j0 = (tile / tiles_k) * TJ, k0 = (tile % tiles_k) * TK;
   const int i0 = chunk * TI;
   const int iend = min(i0 + TI, g.nx);
@@ -820,6 +847,7 @@ static void tiled_go(const Dims &g, int R, const T *E, const ModeC<T> &mc, const
   // vector still in the 256 MB last-level cache (one 64^3 cell in FP64, 38
   // MB, solves as fast either way)
   OpArgs<T> an = a;
+  an.spread = spread_rule(a.spread, tiles * chunks);
   an.nt = (size_t)R * 3 * (size_t)g.V * sizeof(T) >= ((size_t)128 << 20) ? 1 : 0;
   if (R % kRHS) throw std::runtime_error("right-hand sides must come in groups of six");
   if (fused &&
@@ -1081,10 +1109,10 @@ template <typename T, int ST, int EP, int NG, int SYM>
 __global__ __launch_bounds__(kBlock) void k_stencil_plane(Dims g, const T *__restrict__ S, OpArgs<T> a,
                                                           int tiles_k, int tiles) {
   constexpr int G = kRHS / NG;  // load-case groups per sample
-  // logical order (cell, plane, tile, group), XCD-contiguous (see xcd_order)
-  const int L = xcd_order(blockIdx.x, gridDim.x);
-  const int grp = L % G, tile = (L / G) % tiles, i = (L / (G * tiles)) % g.nx;
-  const int smp = L / (G * tiles * g.nx), lc0 = grp * NG;
+  // units of (plane, tile), the groups of a unit next to each other
+  const WorkId id = work_order(blockIdx.x, gridDim.x, gridDim.x / (G * tiles * g.nx), tiles * g.nx, G, a.spread);
+  const int tile = id.unit % tiles, i = id.unit / tiles;
+  const int smp = id.cell, lc0 = id.inner * NG;
   unsigned mask = 0;
 #pragma unroll
   for (int t = 0; t < NG; t++) mask |= a.act[smp * kRHS + lc0 + t] ? (1u << t) : 0u;
@@ -1239,7 +1267,7 @@ __global__ __launch_bounds__(kBlock) void k_stencil_plane(Dims g, const T *__res
 
 template <typename T>
 void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpArgs<T> &a,
-                    hipStream_t s) {
+                    hipStream_t s, int cells) {
   const int blocks = (g.V + kBlock - 1) / kBlock;
   const int nsmp = (R + kRHS - 1) / kRHS;
   const int sym = (g.nx > 2 && g.ny > 2 && g.nz > 2) ? 1 : 0;
@@ -1251,19 +1279,22 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   const int tiles_k = (g.nz + kTile - 1) / kTile, tiles_j = (g.ny + kTile - 1) / kTile;
   const long pl_blocks = (long)tiles_j * tiles_k * g.nx * nsmp * (kRHS / NG);
   // (and a sample's stencil addressable by a buffer resource: < 2 GiB)
-  const bool plane = g.ny >= kTile && g.nz >= kTile && g.nx >= 3 && R % kRHS == 0 && pl_blocks >= 256 &&
+  const long pl_live = pl_blocks / nsmp * cells;
+  const bool plane = g.ny >= kTile && g.nz >= kTile && g.nx >= 3 && R % kRHS == 0 && pl_live >= 256 &&
                      (size_t)243 * g.V * sizeof(T) < ((size_t)1 << 31);
   // all load cases per thread once that still leaves >= 2 workgroups per CU
-  const bool multi = (long)blocks * nsmp >= 512 && R % kRHS == 0;
+  const bool multi = (long)blocks * cells >= 512 && R % kRHS == 0;
   const int split_blocks = (g.V + kSplitNodes - 1) / kSplitNodes;
+  OpArgs<T> an = a;
+  an.spread = spread_rule(a.spread, tiles_j * tiles_k * g.nx);
 #define GO(S_, E_)                                                                               \
   if (st == S_ && ep == E_) {                                                                    \
     if (plane && sym)                                                                            \
       hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG, 1>), dim3((unsigned)pl_blocks), dim3(kBlock), \
-                         0, s, g, S, a, tiles_k, tiles_j * tiles_k);                             \
+                         0, s, g, S, an, tiles_k, tiles_j * tiles_k);                            \
     else if (plane)                                                                              \
       hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG, 0>), dim3((unsigned)pl_blocks), dim3(kBlock), \
-                         0, s, g, S, a, tiles_k, tiles_j * tiles_k);                             \
+                         0, s, g, S, an, tiles_k, tiles_j * tiles_k);                            \
     else if (multi)                                                                              \
       hipLaunchKernelGGL((k_stencil<T, S_, E_>), dim3(blocks, nsmp), dim3(kBlock), 0, s, g, S,       \
                          a, sym);                                                                \
@@ -1306,7 +1337,7 @@ void launch_add2(int V, int R, const T *xn, const T *d, T *x, const int *act, hi
   template void launch_tiled<T>(int, int, const Dims &, int, const T *, const ModeCoef &,       \
                                 const OpArgs<T> &, hipStream_t, int, hipEvent_t, hipEvent_t);   \
   template void launch_stencil<T>(int, int, const Dims &, int, const T *, const OpArgs<T> &,    \
-                                  hipStream_t);                                                 \
+                                  hipStream_t, int);                                            \
   template void launch_add2<T>(int, int, const T *, const T *, T *, const int *, hipStream_t);
 
 FEMH_OPS_INST(double)

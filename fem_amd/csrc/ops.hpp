@@ -80,6 +80,9 @@ struct OpArgs {
   // outputs stored non-temporally (set by the fine-level launcher for
   // vectors too large to stay in the caches until the next launch reads them)
   int nt = 0;
+  // in: the launch is sized for a few remaining right-hand sides; set by the
+  // launchers to the workgroup order (work_order in ops.hip)
+  int spread = 0;
 };
 
 // fine level (tiled cube-mode voxel kernel).  shape: launch shape, bits 0-7
@@ -106,10 +109,11 @@ int tiled_slabs(const Dims &g, int R, int shape, int sz);
 // it is when its planes are pinned)
 int tiled_sparse_shape(const Dims &g, int R, int Ract, int shape, int sz);
 
-// coarse level (27-point block stencil, one RHS per thread)
+// coarse level (27-point block stencil, one RHS per thread).  cells: the cells
+// the launch is sized for (at most R / 6; the others are expected inactive)
 template <typename T>
 void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpArgs<T> &a,
-                    hipStream_t s);
+                    hipStream_t s, int cells);
 
 // x = xn + d
 template <typename T>

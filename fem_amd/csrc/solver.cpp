@@ -243,6 +243,7 @@ template <typename T>
 void Context::op(Hierarchy<T> &h, int l, int st, int ep, OpArgs<T> a) {
   const Level<T> &L = h.lv[l];
   if (!a.Dinv) a.Dinv = L.Dinv.template as<T>();
+  a.spread = live_rhs > 0;
   if (l == 0) {
     const Dims &g0 = L.g;
     const bool dense = o.apply_kernel == 1 && st == ST_PLAIN && (ep == EP_AX || ep == EP_AXD || ep == EP_RES);
@@ -288,7 +289,7 @@ void Context::op(Hierarchy<T> &h, int l, int st, int ep, OpArgs<T> a) {
       launch(nullptr, nullptr);
     }
   } else {
-    launch_stencil<T>(st, ep, L.g, R, L.S.template as<T>(), a, stream);
+    launch_stencil<T>(st, ep, L.g, R, L.S.template as<T>(), a, stream, live_cells());
   }
 }
 
@@ -768,7 +769,7 @@ bool Context::post_smooth(Hierarchy<T> &h, int l, const T *bb, T *xx, const int 
   } else {
     // (out of place: the smoothing step stages xn and writes xx)
     T *xn = L.xn.template as<T>();
-    launch_prolong_add<T>(L.g, C.g, R, C.x.template as<T>(), xx, act_, stream, xn, xfer_shape(l));
+    launch_prolong_add<T>(L.g, C.g, R, C.x.template as<T>(), xx, act_, stream, xn, xfer_planes(l));
     a.u = xn;
     op<T>(h, l, ST_PLAIN, first, a);
   }
@@ -815,7 +816,7 @@ bool Context::vcycle(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_
       cheb_run<T>(h, l, bb, xx, act_, nu_pre(l), o.cheby_ratio);
       apply<T>(h, l, xx, L.r.template as<T>(), bb, 1, act_, nullptr, 0);
     }
-    launch_restrict<T>(L.g, C.g, R, L.r.template as<T>(), C.b.template as<T>(), act_, stream, xfer_shape(l));
+    launch_restrict<T>(L.g, C.g, R, L.r.template as<T>(), C.b.template as<T>(), act_, stream, xfer_planes(l));
   }
   vcycle<T>(h, l + 1, C.b.template as<T>(), C.x.template as<T>(), act_, -1);
   return post_smooth<T>(h, l, bb, xx, act_, dot_slot);
@@ -870,7 +871,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   if (!nact) return;
   set_act(A_PCG, active);
   const int *ap = actp(A_PCG);
-  const int np_rz = jac ? vec_parts(V) : rz_parts(h);
+  int np_rz = jac ? vec_parts(V) : rz_parts(h);
   // z_ready: the caller already left z = M^-1 b and r.z in S_RZ0
   if (!z_ready) precond<T>(h, rv, zv, ap, S_RZ0);
   // Fine-level tiled operator: the direction update p = z + beta p runs
@@ -928,18 +929,19 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
       launch_p_update<T>(V, R, pv, zv, rzn, rzc, 0, ap, red, np_rz, stream, lz_beta, cnt);
   };
   std::vector<int> hact(kMaxR), hst(kMaxR);
+  int nlive = nact;
   // host look at the device state: false when no right-hand side is left.
   // Only k_pcg_check clears a right-hand side's activity, and it sets the
   // state (1 or 2) when it does, so the state alone tells which are left.
   auto poll = [&]() {
     FEMH_HIP(hipMemcpyAsync(hst.data(), pst, sizeof(int) * R, hipMemcpyDeviceToHost, stream));
     FEMH_HIP(hipStreamSynchronize(stream));
-    bool any = false;
+    nlive = 0;
     for (int t = 0; t < R; t++) {
       if (hst[t] == 2) throw Error(FEMH_NONFINITE, "residual became non-finite");
-      any = any || (active[t] != 0 && hst[t] == 0);
+      nlive += active[t] != 0 && hst[t] == 0;
     }
-    return any;
+    return nlive > 0;
   };
   // Iterations 2k and 2k+1 use the same buffers and slots (ping-pong of the
   // direction and of the r.z parity), so with graphs on, the pair is
@@ -951,12 +953,12 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   bool live = it < max_iter ? poll() : false;
   const bool graphs = o.graph && !prof;
   hipGraphExec_t exec = nullptr;
-  if (graphs && live && max_iter - it >= 2) {
+  auto record = [&]() {
     GraphKey key{};
     key.v = {(long long)sizeof(T), (long long)R, (long long)(uintptr_t)xv, (long long)(uintptr_t)rv,
              (long long)(uintptr_t)zv, (long long)(uintptr_t)pv, (long long)(uintptr_t)qv,
              (long long)(uintptr_t)lz_alpha, (long long)(uintptr_t)h.cheb.p, (long long)h.lv.size(),
-             (long long)h.ndense, (long long)shape_fine, (long long)xfer_hash(), (long long)z_ready,
+             (long long)h.ndense, (long long)shape_fine | (long long)live_rhs << 32, (long long)xfer_hash(), (long long)z_ready,
              hier_hash(h)};
     std::memcpy(&key.tol, &tol, sizeof(double));
     exec = find_graph(key);
@@ -978,8 +980,41 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
       FEMH_HIP(ie);
       graphs_.push_back({key, exec});
     }
-  }
+  };
+  if (graphs && live && max_iter - it >= 2) record();
+  // A long solve that is down to a quarter of its right-hand sides or fewer:
+  // launches sized for all of them then leave each remaining one to a few
+  // workgroups that march through 32 planes (48^3, 12 binary cells, one hard
+  // cell left: 55-70 us a fine launch, and it was left for 400 of 470
+  // iterations).  From kSparseAfter iterations on, the launches are sized for
+  // the next of R/4, R/16, .. that covers those left.  Solves of ordinary
+  // length never get there, so they pay no second recording.
+  struct Restore {
+    Context &c;
+    int shape;
+    ~Restore() {
+      c.shape_fine = shape;
+      c.live_rhs = 0;
+    }
+  } restore{*this, shape_fine};
+  constexpr int kSparseAfter = 24;
+  auto resize = [&]() {
+    if (jac || o.apply_kernel == 1 || it < kSparseAfter || !live) return;
+    int q = live_rhs > 0 ? live_rhs : R;
+    const int was = q;
+    while (q / 4 >= nlive) q /= 4;
+    if (q == was) return;
+    const int np_old = np_rz;
+    live_rhs = q;
+    shape_fine = tiled_sparse_shape(g, R, q, restore.shape, (int)sizeof(T));
+    np_rz = rz_parts(h);
+    // r . z of the last iteration, in the old launch's partials, as one partial
+    launch_collapse(R, (it & 1) ? S_RZ1 : S_RZ0, red, np_old, np_rz, stream);
+    FEMH_HIP(hipGetLastError());
+    if (graphs && max_iter - it >= 2) record();
+  };
   while (live && it < max_iter) {
+    resize();
     if (exec && max_iter - it >= 2) {
       FEMH_HIP(hipGraphLaunch(exec, stream));
       it += 2;

@@ -186,6 +186,11 @@ struct Context {
   int shape_fine = 0;
   std::vector<int> shape_xfer;
   int xfer_shape(int l) const { return l < (int)shape_xfer.size() ? shape_xfer[l] : 0; }
+  // right-hand sides that the launches of the running PCG are sized for (0:
+  // all R); pcg lowers it when a long solve is down to a few (see there)
+  int live_rhs = 0;
+  int live_cells() const { return live_rhs > 0 && live_rhs < nb ? live_rhs : nb; }
+  int xfer_planes(int l) const { return live_rhs > 0 ? 1 : xfer_shape(l); }
   template <typename T>
   void autotune(Hierarchy<T> &h);
 
