@@ -347,7 +347,8 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   constexpr bool kStD = ST == ST_DSCALE || ST == ST_DPROLONG;  // stages b / (theta D)
   constexpr int CJ = TJ / 2 + 2, CK = TK / 2 + 2;              // coarse nodes around the tile (kProl)
   constexpr unsigned SZ = sizeof(T);
-  const WorkId id = work_order(blockIdx.x, gridDim.x, gridDim.x / (kRHS * tiles * chunks), tiles * chunks, kRHS, a.spread);
+  const int inner = EP == EP_AXD ? 1 : kRHS;  // (the power iteration runs load case 0 only)
+  const WorkId id = work_order(blockIdx.x, gridDim.x, gridDim.x / (inner * tiles * chunks), tiles * chunks, inner, a.spread);
   const int smp = id.cell, tile = id.unit % tiles, chunk = id.unit / tiles;
   const int r = smp * kRHS + id.inner;
   if (!a.act[r]) return;
@@ -855,14 +856,15 @@ static void tiled_go(const Dims &g, int R, const T *E, const ModeC<T> &mc, const
     throw std::runtime_error("fused grid transfers need the halved grid and chunks of even length");
   // buffer resources address a right-hand side's vector with 32-bit offsets
   if ((size_t)3 * g.V * sizeof(T) >= ((size_t)1 << 31)) throw std::runtime_error("grid too large for the tiled operator");
+  const int grid = tiles * chunks * (EP == EP_AXD ? R / kRHS : R);
   if (ev0) {
     // timed launch: the runtime records the events at the kernel's own start
     // and end, so no queue gap is counted
-    hipExtLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, ev0, ev1,
+    hipExtLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(grid), dim3(TJ * TK), 0, s, ev0, ev1,
                           0, g, E, mc, an, TI, tiles_k, tiles, chunks);
     return;
   }
-  hipLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(tiles * chunks * R), dim3(TJ * TK), 0, s, g, E, mc, an,
+  hipLaunchKernelGGL((k_tiled<T, ST, EP, TJ, TK, EP == EP_PRE>), dim3(grid), dim3(TJ * TK), 0, s, g, E, mc, an,
                      TI, tiles_k, tiles, chunks);
 }
 
@@ -1034,7 +1036,7 @@ constexpr int kSplitNodes = 64, kSplitWaves = 9;
 template <typename T, int ST, int EP>
 __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims g, const T *__restrict__ S,
                                                                              OpArgs<T> a, int sym) {
-  const int r = blockIdx.y;
+  const int r = EP == EP_AXD ? (int)blockIdx.y * kRHS : (int)blockIdx.y;
   if (!a.act[r]) return;
   const int smp = r / kRHS, lane = threadIdx.x % kSplitNodes, w = threadIdx.x / kSplitNodes;
   const int n = blockIdx.x * kSplitNodes + lane;
@@ -1046,6 +1048,15 @@ __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims
   const size_t off = (size_t)r * 3 * V;
   __shared__ T part[kSplitWaves][3][kSplitNodes];
   T acc[3] = {0, 0, 0};
+  // (wave 0 finishes the nodes: what its epilogue reads is asked for first, so
+  // that it arrives with the stencil row and not after it)
+  EpiIn<T> pin;
+  T uo[3];
+  if (w == 0 && live) {
+    epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
+#pragma unroll
+    for (int c = 0; c < 3; c++) uo[c] = stage_at<T, ST>(a, Ds, ti, off, V, c, n);
+  }
   if (live) {
     int i, j, k;
     node_ijk(g, n, i, j, k);
@@ -1071,19 +1082,16 @@ __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims
   for (int c = 0; c < 3; c++) part[w][c][lane] = acc[c];
   __syncthreads();
   if (w != 0 || !live) return;
-  T Au[3], uo[3];
+  T Au[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     T s = part[0][c][lane];
 #pragma unroll
     for (int q = 1; q < kSplitWaves; q++) s += part[q][c][lane];
     Au[c] = s;
-    uo[c] = stage_at<T, ST>(a, Ds, ti, off, V, c, n);
   }
   const T c1 = a.cheb ? (T)a.cheb[kMaxB + smp] : (T)0, c2 = a.cheb ? (T)a.cheb[2 * kMaxB + smp] : (T)0;
   DotAcc dv;
-  EpiIn<T> pin;
-  epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
   epilogue<T, ST, EP>(a, pin, ti, c1, c2, off, V, n, Au, uo, dv);
 }
 
@@ -1108,7 +1116,7 @@ constexpr int kStBatch = 3;  // stencil blocks whose coefficient loads are issue
 template <typename T, int ST, int EP, int NG, int SYM>
 __global__ __launch_bounds__(kBlock) void k_stencil_plane(Dims g, const T *__restrict__ S, OpArgs<T> a,
                                                           int tiles_k, int tiles) {
-  constexpr int G = kRHS / NG;  // load-case groups per sample
+  constexpr int G = EP == EP_AXD ? 1 : kRHS / NG;  // load-case groups per sample
   // units of (plane, tile), the groups of a unit next to each other
   const WorkId id = work_order(blockIdx.x, gridDim.x, gridDim.x / (G * tiles * g.nx), tiles * g.nx, G, a.spread);
   const int tile = id.unit % tiles, i = id.unit / tiles;
@@ -1274,32 +1282,49 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   // planes of at least one full 16x16 tile: the one-plane LDS kernel (all six
   // load cases of a sample per workgroup in FP32, 47 KB of LDS: the stencil
   // row is read once per node; three in FP64), once that gives a workgroup
-  // per CU
-  constexpr int NG = sizeof(T) == 4 ? kRHS : kRHS / 2;
+  // per CU.  One cell, and FP64 in general, take it with three load cases per
+  // workgroup from 192 workgroups on: the nine-wave split kernel below re-reads
+  // the row for every load case (a smoothing step of one cell: FP32 32^3, 17.3
+  // -> 9.7 us; FP64 30 x 22 x 26, 240 workgroups, 30.8 -> 13.6 us).  The power
+  // iteration runs one load case.
   const int tiles_k = (g.nz + kTile - 1) / kTile, tiles_j = (g.ny + kTile - 1) / kTile;
-  const long pl_blocks = (long)tiles_j * tiles_k * g.nx * nsmp * (kRHS / NG);
+  const long units = (long)tiles_j * tiles_k * g.nx;
   // (and a sample's stencil addressable by a buffer resource: < 2 GiB)
-  const long pl_live = pl_blocks / nsmp * cells;
-  const bool plane = g.ny >= kTile && g.nz >= kTile && g.nx >= 3 && R % kRHS == 0 && pl_live >= 256 &&
-                     (size_t)243 * g.V * sizeof(T) < ((size_t)1 << 31);
+  const bool fits = g.ny >= kTile && g.nz >= kTile && g.nx >= 3 && R % kRHS == 0 &&
+                    (size_t)243 * g.V * sizeof(T) < ((size_t)1 << 31);
+  int ng = 0;  // load cases per workgroup of the one-plane kernel (0: not taken)
+  if (fits && sizeof(T) == 4 && units * cells >= 256)
+    ng = kRHS;
+  else if (fits && (sizeof(T) == 8 || nsmp == 1) && units * cells * 2 >= 192)
+    ng = kRHS / 2;
+  const unsigned pl_blocks = ng ? (unsigned)(units * nsmp * (kRHS / ng)) : 0u;
   // all load cases per thread once that still leaves >= 2 workgroups per CU
   const bool multi = (long)blocks * cells >= 512 && R % kRHS == 0;
   const int split_blocks = (g.V + kSplitNodes - 1) / kSplitNodes;
   OpArgs<T> an = a;
-  an.spread = spread_rule(a.spread, tiles_j * tiles_k * g.nx);
+  an.spread = spread_rule(a.spread, (int)units);
+#define PLANE(S_, E_, NG_, SYM_, GRID_)                                                             \
+  hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG_, SYM_>), dim3(GRID_), dim3(kBlock), 0, s, g, S, an, tiles_k, \
+                     tiles_j *tiles_k)
 #define GO(S_, E_)                                                                               \
   if (st == S_ && ep == E_) {                                                                    \
-    if (plane && sym)                                                                            \
-      hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG, 1>), dim3((unsigned)pl_blocks), dim3(kBlock), \
-                         0, s, g, S, an, tiles_k, tiles_j * tiles_k);                            \
-    else if (plane)                                                                              \
-      hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG, 0>), dim3((unsigned)pl_blocks), dim3(kBlock), \
-                         0, s, g, S, an, tiles_k, tiles_j * tiles_k);                            \
-    else if (multi)                                                                              \
+    if constexpr (E_ == EP_AXD) {                                                                \
+      if (ng && sym) PLANE(S_, E_, 1, 1, (unsigned)(units * nsmp));                              \
+      else if (ng) PLANE(S_, E_, 1, 0, (unsigned)(units * nsmp));                                \
+    } else {                                                                                     \
+      if constexpr (sizeof(T) == 4) {                                                            \
+        if (ng == kRHS && sym) PLANE(S_, E_, kRHS, 1, pl_blocks);                                \
+        else if (ng == kRHS) PLANE(S_, E_, kRHS, 0, pl_blocks);                                  \
+      }                                                                                          \
+      if (ng == kRHS / 2 && sym) PLANE(S_, E_, kRHS / 2, 1, pl_blocks);                          \
+      else if (ng == kRHS / 2) PLANE(S_, E_, kRHS / 2, 0, pl_blocks);                            \
+    }                                                                                            \
+    if (ng) return;                                                                              \
+    if (multi)                                                                                   \
       hipLaunchKernelGGL((k_stencil<T, S_, E_>), dim3(blocks, nsmp), dim3(kBlock), 0, s, g, S,       \
                          a, sym);                                                                \
     else                                                                                         \
-      hipLaunchKernelGGL((k_stencil_split<T, S_, E_>), dim3(split_blocks, R),                       \
+      hipLaunchKernelGGL((k_stencil_split<T, S_, E_>), dim3(split_blocks, E_ == EP_AXD ? nsmp : R), \
                          dim3(kSplitNodes * kSplitWaves), 0, s, g, S, a, sym);                   \
     return;                                                                                      \
   }
@@ -1314,6 +1339,7 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   GO(ST_PLAIN, EP_CHEB0)
   GO(ST_PLAIN, EP_FIN1)
 #undef GO
+#undef PLANE
   throw std::runtime_error("no operator kernel for this stage/epilogue pair");
 }
 

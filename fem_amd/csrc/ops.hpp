@@ -15,7 +15,8 @@
 // staged value there:
 //   EP_AX       y = Au            (optional FP64 partial of u . Au; with ST_PUPD,
 //                                  pout = u_own: the new PCG direction)
-//   EP_AXD      y = Au / D        (a power-iteration step)
+//   EP_AXD      y = Au / D        (a power-iteration step: load case 0 of every
+//                                  cell, the only one launched)
 //   EP_RES      y = b - Au        (optional FP64 partials of r.r, b.u, u.r)
 //   EP_PRE      b - Au ; on the fine level restricted to y = P^T (b - Au) on the
 //               coarse grid gc, on the coarse levels y = b - Au itself
