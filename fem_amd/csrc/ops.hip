@@ -1025,37 +1025,44 @@ __global__ __launch_bounds__(kBlock) void k_stencil(Dims g, const T *__restrict_
 }
 
 // Small levels (a few thousand nodes: too few threads to cover the latency of
-// a node's 27 dependent block loads): one right-hand side per workgroup row
+// a node's 27 dependent block loads): NR right-hand sides per workgroup row
 // (blockIdx.y) and 64 consecutive nodes per workgroup, whose stencil rows are
 // split over nine waves -- wave w = 3 di + dj applies the three blocks
 // (di, dj, 0..2) -- so a thread's load chain is three blocks long.  The nine
-// partial sums meet in LDS and wave 0 finishes the node.  Same block order
-// and symmetric reads as stencil_node; only the summation order differs.
+// partial sums meet in LDS and wave t finishes the nodes of right-hand side t.
+// Same block order and symmetric reads as stencil_node; only the summation
+// order differs.
 constexpr int kSplitNodes = 64, kSplitWaves = 9;
 
-template <typename T, int ST, int EP>
+template <typename T, int ST, int EP, int NR>
 __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims g, const T *__restrict__ S,
                                                                              OpArgs<T> a, int sym) {
-  const int r = EP == EP_AXD ? (int)blockIdx.y * kRHS : (int)blockIdx.y;
-  if (!a.act[r]) return;
-  const int smp = r / kRHS, lane = threadIdx.x % kSplitNodes, w = threadIdx.x / kSplitNodes;
+  const int r0 = EP == EP_AXD ? (int)blockIdx.y * kRHS : (int)blockIdx.y * NR;
+  unsigned mask = 0;
+#pragma unroll
+  for (int t = 0; t < NR; t++) mask |= a.act[r0 + t] ? (1u << t) : 0u;
+  if (!mask) return;
+  const int smp = r0 / kRHS, lane = threadIdx.x % kSplitNodes, w = threadIdx.x / kSplitNodes;
   const int n = blockIdx.x * kSplitNodes + lane;
   const bool live = n < g.V;
   const int V = g.V;
   const T *__restrict__ Ss = S + (size_t)smp * 243 * V;
   const T *__restrict__ Ds = a.Dinv ? a.Dinv + (size_t)smp * 3 * V : nullptr;
   const T ti = a.cheb ? (T)a.cheb[smp] : (T)0;
-  const size_t off = (size_t)r * 3 * V;
-  __shared__ T part[kSplitWaves][3][kSplitNodes];
-  T acc[3] = {0, 0, 0};
-  // (wave 0 finishes the nodes: what its epilogue reads is asked for first, so
-  // that it arrives with the stencil row and not after it)
+  const size_t off0 = (size_t)r0 * 3 * V, offw = off0 + (size_t)w * 3 * V;
+  __shared__ T part[NR][kSplitWaves][3][kSplitNodes];
+  T acc[NR][3];
+#pragma unroll
+  for (int t = 0; t < NR; t++) acc[t][0] = acc[t][1] = acc[t][2] = 0;
+  // (wave t finishes right-hand side t: what its epilogue reads is asked for
+  // first, so that it arrives with the stencil row and not after it)
+  const bool fin = w < NR && live && ((mask >> w) & 1u);
   EpiIn<T> pin;
   T uo[3];
-  if (w == 0 && live) {
-    epi_load<T, ST, EP>(a, Ds, off, V, n, pin);
+  if (fin) {
+    epi_load<T, ST, EP>(a, Ds, offw, V, n, pin);
 #pragma unroll
-    for (int c = 0; c < 3; c++) uo[c] = stage_at<T, ST>(a, Ds, ti, off, V, c, n);
+    for (int c = 0; c < 3; c++) uo[c] = stage_at<T, ST>(a, Ds, ti, offw, V, c, n);
   }
   if (live) {
     int i, j, k;
@@ -1071,28 +1078,35 @@ __global__ __launch_bounds__(kSplitNodes *kSplitWaves) void k_stencil_split(Dims
         load_block(Ss, 26 - o, V, nb, true, sv);
       else
         load_block(Ss, o, V, n, false, sv);
-      const T u0 = stage_at<T, ST>(a, Ds, ti, off, V, 0, nb), u1 = stage_at<T, ST>(a, Ds, ti, off, V, 1, nb),
-              u2 = stage_at<T, ST>(a, Ds, ti, off, V, 2, nb);
-      acc[0] += sv[0] * u0 + sv[1] * u1 + sv[2] * u2;
-      acc[1] += sv[3] * u0 + sv[4] * u1 + sv[5] * u2;
-      acc[2] += sv[6] * u0 + sv[7] * u1 + sv[8] * u2;
+#pragma unroll
+      for (int t = 0; t < NR; t++) {
+        if (NR > 1 && !((mask >> t) & 1u)) continue;
+        const size_t off = off0 + (size_t)t * 3 * V;
+        const T u0 = stage_at<T, ST>(a, Ds, ti, off, V, 0, nb), u1 = stage_at<T, ST>(a, Ds, ti, off, V, 1, nb),
+                u2 = stage_at<T, ST>(a, Ds, ti, off, V, 2, nb);
+        acc[t][0] += sv[0] * u0 + sv[1] * u1 + sv[2] * u2;
+        acc[t][1] += sv[3] * u0 + sv[4] * u1 + sv[5] * u2;
+        acc[t][2] += sv[6] * u0 + sv[7] * u1 + sv[8] * u2;
+      }
     }
   }
 #pragma unroll
-  for (int c = 0; c < 3; c++) part[w][c][lane] = acc[c];
+  for (int t = 0; t < NR; t++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) part[t][w][c][lane] = acc[t][c];
   __syncthreads();
-  if (w != 0 || !live) return;
+  if (!fin) return;
   T Au[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    T s = part[0][c][lane];
+    T s = part[w][0][c][lane];
 #pragma unroll
-    for (int q = 1; q < kSplitWaves; q++) s += part[q][c][lane];
+    for (int q = 1; q < kSplitWaves; q++) s += part[w][q][c][lane];
     Au[c] = s;
   }
   const T c1 = a.cheb ? (T)a.cheb[kMaxB + smp] : (T)0, c2 = a.cheb ? (T)a.cheb[2 * kMaxB + smp] : (T)0;
   DotAcc dv;
-  epilogue<T, ST, EP>(a, pin, ti, c1, c2, off, V, n, Au, uo, dv);
+  epilogue<T, ST, EP>(a, pin, ti, c1, c2, offw, V, n, Au, uo, dv);
 }
 
 // One-plane form of the tiled stencil kernel, for levels with planes of at
@@ -1301,6 +1315,11 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   // all load cases per thread once that still leaves >= 2 workgroups per CU
   const bool multi = (long)blocks * cells >= 512 && R % kRHS == 0;
   const int split_blocks = (g.V + kSplitNodes - 1) / kSplitNodes;
+  // two right-hand sides per split workgroup once one each gives a workgroup
+  // per CU: they share the stencil row, which every right-hand side otherwise
+  // reads from L2 again (16^3, one cell in FP64, 384 workgroups: 7.0 -> 5.7 us a
+  // step; three per workgroup, 128 left: 6.6 us)
+  const int nr = R % kRHS == 0 && (long)split_blocks * cells * kRHS >= 256 ? 2 : 1;
   OpArgs<T> an = a;
   an.spread = spread_rule(a.spread, (int)units);
 #define PLANE(S_, E_, NG_, SYM_, GRID_)                                                             \
@@ -1323,8 +1342,11 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
     if (multi)                                                                                   \
       hipLaunchKernelGGL((k_stencil<T, S_, E_>), dim3(blocks, nsmp), dim3(kBlock), 0, s, g, S,       \
                          a, sym);                                                                \
+    else if (E_ == EP_AXD || nr == 1)                                                            \
+      hipLaunchKernelGGL((k_stencil_split<T, S_, E_, 1>), dim3(split_blocks, E_ == EP_AXD ? nsmp : R), \
+                         dim3(kSplitNodes * kSplitWaves), 0, s, g, S, a, sym);                   \
     else                                                                                         \
-      hipLaunchKernelGGL((k_stencil_split<T, S_, E_>), dim3(split_blocks, E_ == EP_AXD ? nsmp : R), \
+      hipLaunchKernelGGL((k_stencil_split<T, S_, E_, 2>), dim3(split_blocks, R / 2),             \
                          dim3(kSplitNodes * kSplitWaves), 0, s, g, S, a, sym);                   \
     return;                                                                                      \
   }
