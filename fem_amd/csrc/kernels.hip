@@ -515,15 +515,28 @@ __global__ __launch_bounds__(kBlock) void k_beta(int rz_new, int rz_old, int fir
 // right-hand side that reaches tol (state 1) or turns non-finite (state 2)
 // leaves the activity array, so the rest of the iteration and later
 // iterations skip it.  cnt counts each right-hand side's iterations.
+// With beta (Jacobi, whose update launch also leaves r.z) it forms the next
+// direction's beta as k_beta does: one launch fewer per iteration.
 __global__ __launch_bounds__(kBlock) void k_pcg_check(int *__restrict__ act, Reduce red, int np,
                                                       const double *__restrict__ bb, double tol,
                                                       int *__restrict__ cnt, double *__restrict__ relres,
-                                                      int *__restrict__ state) {
+                                                      int *__restrict__ state, int rz_new, int rz_old,
+                                                      double *__restrict__ beta, double *__restrict__ beta_out) {
   const int rr = blockIdx.x;
   if (!act[rr]) return;
   const double s = sum_parts(red, S_RR, rr, np);
+  double den = 0, num = 0;
+  if (beta) {
+    den = sum_parts(red, rz_old, rr, np);
+    num = sum_parts(red, rz_new, rr, np);
+  }
   if (threadIdx.x == 0) {
     cnt[rr] += 1;
+    if (beta) {
+      const double b = den != 0.0 ? num / den : 0.0;
+      beta[rr] = b;
+      if (beta_out) beta_out[(size_t)(cnt[rr] - 1) * kMaxR + rr] = b;
+    }
     if (!(s <= 1.7976931348623157e308) || s != s) {
       state[rr] = 2;
       act[rr] = 0;
@@ -1053,8 +1066,10 @@ void launch_p_update(int V, int R, T *p, const T *z, int rz_new, int rz_old, int
                      first, act, red, np_rz, beta_out, cnt);
 }
 void launch_pcg_check(int R, int *act, const Reduce &red, int np, const double *bb, double tol, int *cnt,
-                      double *relres, int *state, hipStream_t s) {
-  hipLaunchKernelGGL(k_pcg_check, dim3(R), dim3(kBlock), 0, s, act, red, np, bb, tol, cnt, relres, state);
+                      double *relres, int *state, hipStream_t s, int rz_new, int rz_old, double *beta,
+                      double *beta_out) {
+  hipLaunchKernelGGL(k_pcg_check, dim3(R), dim3(kBlock), 0, s, act, red, np, bb, tol, cnt, relres, state, rz_new,
+                     rz_old, beta, beta_out);
 }
 void launch_permute_case(int n, int nb, double *x, int src, int dst, int swap, unsigned mask, hipStream_t s) {
   hipLaunchKernelGGL(k_permute_case, dim3(grid_for(n * n * n), nb), dim3(kBlock), 0, s, n, x, src, dst, swap,

@@ -167,7 +167,8 @@ void launch_beta(int R, int rz_new, int rz_old, int first, const int *act, const
 // partials of S_RR; relres <= tol clears act (state 1), a non-finite r.r too
 // (state 2)
 void launch_pcg_check(int R, int *act, const Reduce &red, int np, const double *bb, double tol, int *cnt,
-                      double *relres, int *state, hipStream_t s);
+                      double *relres, int *state, hipStream_t s, int rz_new = 0, int rz_old = 0, double *beta = nullptr,
+                      double *beta_out = nullptr);
 // cubic structure: load case dst from load case src by an axis swap of the
 // cube grid (swap 0: x <-> y, 1: x <-> z), points and displacement components
 // alike, for the samples s with bit s of mask set

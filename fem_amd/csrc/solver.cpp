@@ -878,7 +878,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // inside the A p launch (staged on the fly, written back by the owner),
   // ping-ponging p between pv and a second buffer since neighbours still
   // read the old direction.  beta comes from a one-block-per-RHS kernel.
-  const bool fuse_p = !jac && o.apply_kernel != 1;
+  const bool fuse_p = o.apply_kernel != 1;
   T *pcur = pv, *pnxt = nullptr;
   if (fuse_p) {
     DBuf &alt = sizeof(T) == 8 ? palt : palt32;
@@ -921,6 +921,12 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     }
     launch_pcg_update<T>(V, R, xv, rv, pcur, qv, jac ? D0 : nullptr, zv, rzc, rzn, ap, red, apply_parts((int)sizeof(T)), np_rz,
                          stream, lz_alpha, cnt);
+    if (jac && fuse_p) {
+      // (the update left z and r.z: the check also forms beta)
+      launch_pcg_check(R, apw, red, np_rr, bb_d, tol, cnt, relres_d, pst, stream, rzn, rzc, beta_d.as<double>(),
+                       lz_beta);
+      return;
+    }
     launch_pcg_check(R, apw, red, np_rr, bb_d, tol, cnt, relres_d, pst, stream);
     if (!jac) precond<T>(h, rv, zv, ap, rzn);
     if (fuse_p)
@@ -947,6 +953,12 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // direction and of the r.z parity), so with graphs on, the pair is
   // recorded once into a hipGraph and replayed; the host looks at the device
   // state after every pair (or every check_every iterations without graphs).
+  // A Jacobi iteration is three short launches (about 20 us at 16^3), of which a
+  // look at the state costs as much as one whole iteration, and an iteration of
+  // converged right-hand sides is three launches that return at once: eight
+  // iterations per replay, and without graphs a look every eighth of the
+  // iterations done (at most eight).
+  const int per_replay = jac ? 8 : 2;
   FEMH_HIP(hipGetLastError());
   int it = 1;
   iteration(0, true);
@@ -966,8 +978,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
       hipGraph_t graph = nullptr;
       FEMH_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
       try {
-        iteration(1, false);
-        iteration(0, false);
+        for (int k = 0; k < per_replay; k++) iteration((k & 1) ^ 1, false);
       } catch (...) {
         hipGraph_t g2 = nullptr;
         (void)hipStreamEndCapture(stream, &g2);
@@ -981,7 +992,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
       graphs_.push_back({key, exec});
     }
   };
-  if (graphs && live && max_iter - it >= 2) record();
+  if (graphs && live && max_iter - it >= per_replay) record();
   // A long solve that is down to a quarter of its right-hand sides or fewer:
   // launches sized for all of them then leave each remaining one to a few
   // workgroups that march through 32 planes (48^3, 12 binary cells, one hard
@@ -1011,19 +1022,20 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     // r . z of the last iteration, in the old launch's partials, as one partial
     launch_collapse(R, (it & 1) ? S_RZ1 : S_RZ0, red, np_old, np_rz, stream);
     FEMH_HIP(hipGetLastError());
-    if (graphs && max_iter - it >= 2) record();
+    if (graphs && max_iter - it >= per_replay) record();
   };
   while (live && it < max_iter) {
     resize();
-    if (exec && max_iter - it >= 2) {
+    if (exec && max_iter - it >= per_replay) {
       FEMH_HIP(hipGraphLaunch(exec, stream));
-      it += 2;
+      it += per_replay;
       live = poll();
       continue;
     }
     iteration(it & 1, false);
     it++;
-    if (it % o.check_every == 0 || it == max_iter) live = poll();
+    const int every = jac ? std::max(o.check_every, std::min(8, it / 8)) : o.check_every;
+    if (it % std::max(every, 1) == 0 || it == max_iter) live = poll();
   }
   if (live) poll();
   // results of the run: iterations and residual per right-hand side, and the
