@@ -417,6 +417,7 @@ int femh_prepare(femh_ctx *ctx, const double *E) {
   return guarded(ctx, [&] {
     ctx->c->load(E, 1, false, true);
     ctx->c->build_hierarchy();
+    ctx->c->check_setup();
   });
 }
 

@@ -614,11 +614,13 @@ __global__ __launch_bounds__(kBlock) void k_zero_rhs(int V, double *__restrict__
   for (int t = blockIdx.x * kBlock + threadIdx.x; t < 3 * V; t += gridDim.x * kBlock) x[off + t] = 0.0;
 }
 
+// the first len values of every period of x (blockIdx.y), the same in each
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_fill_hash(size_t n, size_t period, T *__restrict__ x,
+__global__ __launch_bounds__(kBlock) void k_fill_hash(size_t len, size_t period, T *__restrict__ x,
                                                       unsigned long long seed) {
-  for (size_t t = blockIdx.x * (size_t)kBlock + threadIdx.x; t < n; t += (size_t)gridDim.x * kBlock) {
-    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (t % period + 1);
+  x += blockIdx.y * period;
+  for (size_t t = blockIdx.x * (size_t)kBlock + threadIdx.x; t < len; t += (size_t)gridDim.x * kBlock) {
+    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (t + 1);
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z ^= z >> 31;
@@ -960,6 +962,100 @@ __global__ __launch_bounds__(kBlock) void k_finalize(Reduce red, int slot, int n
   if (threadIdx.x == 0) red.scalars[slot * kSlotWidth + blockIdx.x] = s;
 }
 
+// three slots' scalars side by side: scalars[slot0][y * kMaxR + idx]
+__global__ __launch_bounds__(kBlock) void k_finalize3(Reduce red, int slot0, int slot1, int slot2, int np) {
+  const int y = blockIdx.y;
+  const double s = sum_parts(red, y == 0 ? slot0 : y == 1 ? slot1 : slot2, blockIdx.x, np);
+  if (threadIdx.x == 0) red.scalars[slot0 * kSlotWidth + y * kMaxR + blockIdx.x] = s;
+}
+
+__global__ void k_set_act(int *act, ActMask m) {
+  const int t = threadIdx.x;
+  if (t < kMaxR) act[t] = (m.w[t >> 5] >> (t & 31)) & 1u;
+}
+
+// Power iteration: squared norms of the last two iterates of every sample's
+// load case 0 (blockIdx.y) on one level, as block partials
+// part[level][0: y_9, 1: y_10][kMaxB][kRedBlocks]
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_power_norms(int V, const T *__restrict__ y9, const T *__restrict__ y10,
+                                                        double *__restrict__ part) {
+  const int s = blockIdx.y;
+  const size_t off = (size_t)s * kRHS * 3 * V;
+  double n9 = 0, n10 = 0;
+  for (int t = blockIdx.x * kBlock + threadIdx.x; t < 3 * V; t += gridDim.x * kBlock) {
+    const double p = (double)y9[off + t], q = (double)y10[off + t];
+    n9 += p * p;
+    n10 += q * q;
+  }
+  n9 = block_sum(n9);
+  n10 = block_sum(n10);
+  if (threadIdx.x == 0) {
+    part[(size_t)s * kRedBlocks + blockIdx.x] = n9;
+    part[(size_t)(kMaxB + s) * kRedBlocks + blockIdx.x] = n10;
+  }
+}
+
+// lambda_max of every level (blockIdx.x) and sample from the power iteration's
+// norms (with part), and the table of Chebyshev coefficients that follows from
+// it: per level, step and interval [lmax / ratio, lmax] 1/theta and (from step 1
+// on) c1 and c2 of the three-term recurrence d_s = c1 d_{s-1} + c2 D^-1 r_s, for
+// every sample.  (No contraction: the same bits as the plain sequence of
+// operations.)
+__global__ __launch_bounds__(kBlock) void k_cheb_setup(int nb, ChebSetup cs, const double *__restrict__ part,
+                                                       double *__restrict__ lm, double *__restrict__ table) {
+#pragma clang fp contract(off)
+  const int l = blockIdx.x;
+  if (part) {
+    for (int s = 0; s < nb; s++) {
+      double n[2];
+      for (int w = 0; w < 2; w++) {
+        const double *p = part + ((size_t)l * 2 * kMaxB + w * kMaxB + s) * kRedBlocks;
+        double v = 0;
+        for (int i = threadIdx.x; i < cs.np[l]; i += kBlock) v += p[i];
+        n[w] = block_sum(v);
+      }
+      if (threadIdx.x == 0) {
+        const double q = n[1] > 0 || n[1] != n[1] ? n[1] : 0.0;
+        lm[l * kMaxB + s] = cs.scale * sqrt(n[0] > 0 ? q / n[0] : 0.0);
+      }
+    }
+    __syncthreads();
+  }
+  const int kind = threadIdx.x / kMaxB, s = threadIdx.x % kMaxB;
+  if (kind > 1) return;
+  double *t = table + ((size_t)l * cs.steps * 2 + kind) * 3 * kMaxB + s;
+  const double hi = s < nb ? lm[l * kMaxB + s] : 1.0, lo = hi / cs.ratio[kind];
+  const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+  double rho = 1.0 / sigma, c1 = 0.0, c2 = 0.0;
+  for (int st = 0; st < cs.steps; st++) {
+    if (st > 0) {
+      const double rn = 1.0 / (2.0 * sigma - rho);
+      c1 = rn * rho;
+      c2 = 2.0 * rn / delta;
+      rho = rn;
+    }
+    t[0] = s < nb ? 1.0 / theta : 0.0;
+    t[kMaxB] = s < nb ? c1 : 0.0;
+    t[2 * kMaxB] = s < nb ? c2 : 0.0;
+    t += (size_t)2 * 3 * kMaxB;
+  }
+}
+
+// out[s] = 1 where a level's lambda_max is not a positive finite number, 2 where
+// the coarsest operator was not positive definite
+__global__ void k_setup_report(int nb, int levels, const double *lm, const int *bad, double *out) {
+  const int s = threadIdx.x;
+  if (s >= nb) return;
+  double v = 0.0;
+  for (int l = 0; l < levels; l++) {
+    const double x = lm[l * kMaxB + s];
+    if (!(x > 0.0) || !isfinite(x)) v = 1.0;
+  }
+  if (v == 0.0 && bad && bad[s]) v = 2.0;
+  out[s] = v;
+}
+
 // partials [0, np_new) of (slot, RHS) = their sum over np_old, then zeros: a
 // reader that sums np_new of them gets the same value
 __global__ __launch_bounds__(kBlock) void k_collapse(Reduce red, int slot, int np_old, int np_new) {
@@ -1109,11 +1205,11 @@ void launch_remove_mean(int V, int R, T *x, const int *act, const Reduce &red, h
                      grid_for(V));
 }
 template <typename T>
-void launch_fill_hash(size_t n, size_t period, T *x, unsigned long long seed, hipStream_t s) {
-  size_t b = (n + kBlock - 1) / kBlock;
-  if (b > 4096) b = 4096;
+void launch_fill_hash(size_t len, size_t period, int n, T *x, unsigned long long seed, hipStream_t s) {
+  size_t b = (len + kBlock - 1) / kBlock;
+  if (b > 512) b = 512;
   if (b < 1) b = 1;
-  hipLaunchKernelGGL(k_fill_hash<T>, dim3((unsigned)b), dim3(kBlock), 0, s, n, period, x, seed);
+  hipLaunchKernelGGL(k_fill_hash<T>, dim3((unsigned)b, n), dim3(kBlock), 0, s, len, period, x, seed);
 }
 template <typename T>
 void launch_scale_by_dinv_norm(int V, int R, T *y, const T *Dinv, const int *act,
@@ -1183,6 +1279,29 @@ void launch_finalize(const Reduce &red, int slot, int nidx, int np, hipStream_t 
   hipLaunchKernelGGL(k_finalize, dim3(nidx), dim3(kBlock), 0, s, red, slot, np);
 }
 
+void launch_finalize3(const Reduce &red, int slot0, int slot1, int slot2, int nidx, int np, hipStream_t s) {
+  hipLaunchKernelGGL(k_finalize3, dim3(nidx, 3), dim3(kBlock), 0, s, red, slot0, slot1, slot2, np);
+}
+
+void launch_set_act(int *act, const ActMask &m, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_act, dim3(1), dim3(128), 0, s, act, m);
+}
+
+template <typename T>
+void launch_power_norms(int V, int nb, int level, const T *y9, const T *y10, double *part, hipStream_t s) {
+  hipLaunchKernelGGL(k_power_norms<T>, dim3(grid_for(3 * V), nb), dim3(kBlock), 0, s, V, y9, y10,
+                     part + (size_t)level * 2 * kMaxB * kRedBlocks);
+}
+
+void launch_cheb_setup(int levels, int nb, const ChebSetup &cs, const double *part, double *lm, double *table,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_cheb_setup, dim3(levels), dim3(kBlock), 0, s, nb, cs, part, lm, table);
+}
+
+void launch_setup_report(int nb, int levels, const double *lm, const int *bad, double *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_setup_report, dim3(1), dim3(64), 0, s, nb, levels, lm, bad, out);
+}
+
 void launch_collapse(int R, int slot, const Reduce &red, int np_old, int np_new, hipStream_t s) {
   hipLaunchKernelGGL(k_collapse, dim3(R), dim3(kBlock), 0, s, red, slot, np_old, np_new);
 }
@@ -1217,7 +1336,8 @@ void reduce_init(Reduce &red, hipStream_t s) {
   template void launch_dot<T>(int, int, const T *, const T *, int, const int *, const Reduce &,   \
                               hipStream_t);                                                       \
   template void launch_remove_mean<T>(int, int, T *, const int *, const Reduce &, hipStream_t);   \
-  template void launch_fill_hash<T>(size_t, size_t, T *, unsigned long long, hipStream_t);                \
+  template void launch_fill_hash<T>(size_t, size_t, int, T *, unsigned long long, hipStream_t);           \
+  template void launch_power_norms<T>(int, int, int, const T *, const T *, double *, hipStream_t);        \
   template void launch_invert<T>(size_t, const T *, T *, hipStream_t);                            \
   template void launch_fill<T>(size_t, T *, T, hipStream_t);                                      \
   template void launch_scale_by_dinv_norm<T>(int, int, T *, const T *, const int *,               \

@@ -89,6 +89,29 @@ struct StencilOp {
 int dense_parts(const Dims &g);  // partials written by a dense dot-apply
 int vec_parts(int V);             // partials of 3V-vector reductions
 void launch_finalize(const Reduce &red, int slot, int nidx, int np, hipStream_t s);
+// three slots of np partials at once: scalars[slot0][y * kMaxR + idx]
+void launch_finalize3(const Reduce &red, int slot0, int slot1, int slot2, int nidx, int np, hipStream_t s);
+// activity flags of kMaxR right-hand sides from a bit mask passed by value (no
+// host copy, so no wait)
+struct ActMask {
+  unsigned w[kMaxR / 32];
+};
+static_assert(kMaxR % 32 == 0, "whole mask words");
+void launch_set_act(int *act, const ActMask &m, hipStream_t s);
+// spectrum set-up on the device: the power iteration's norms of a level, then
+// lambda_max and the Chebyshev table of all levels, then a flag per sample
+constexpr int kMaxLevels = 32;
+struct ChebSetup {
+  int np[kMaxLevels];  // partials of each level's norms
+  int steps;           // table steps per level and interval
+  double ratio[2];     // intervals [lmax / ratio, lmax]
+  double scale;        // safety factor on the power iteration's estimate
+};
+template <typename T>
+void launch_power_norms(int V, int nb, int level, const T *y9, const T *y10, double *part, hipStream_t s);
+void launch_cheb_setup(int levels, int nb, const ChebSetup &cs, const double *part, double *lm, double *table,
+                       hipStream_t s);
+void launch_setup_report(int nb, int levels, const double *lm, const int *bad, double *out, hipStream_t s);
 // the np_old partials of every RHS as one partial followed by np_new - 1 zeros
 void launch_collapse(int R, int slot, const Reduce &red, int np_old, int np_new, hipStream_t s);
 
@@ -192,9 +215,10 @@ void launch_add_f32_to_f64(int V, int R, const float *d, double *x, const int *a
 // subtract each RHS/component mean (slot S_AUX)
 template <typename T>
 void launch_remove_mean(int V, int R, T *x, const int *act, const Reduce &red, hipStream_t s);
-// x[t] = hash(seed, t mod period) in [-1/2, 1/2)
+// n periods of x: their first len values = hash(seed, t) in [-1/2, 1/2), the
+// same in every period
 template <typename T>
-void launch_fill_hash(size_t n, size_t period, T *x, unsigned long long seed, hipStream_t s);
+void launch_fill_hash(size_t len, size_t period, int n, T *x, unsigned long long seed, hipStream_t s);
 // y *= Dinv and ||y||^2 -> S_AUX[q] (the D^-1 of a power-iteration step on
 // the dense fine-apply path)
 template <typename T>

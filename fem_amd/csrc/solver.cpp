@@ -170,12 +170,22 @@ Context::~Context() {
 }
 
 void Context::set_act(int slot, const std::vector<int> &v) {
-  int h[kMaxR] = {0};
-  for (size_t t = 0; t < v.size() && t < (size_t)kMaxR; t++) h[t] = v[t] ? 1 : 0;
-  // pageable source: the copy completes before the call returns, so the
-  // stack buffer may go away afterwards
-  FEMH_HIP(hipMemcpyAsync(act.as<int>() + slot * kMaxR, h, sizeof(h), hipMemcpyHostToDevice, stream));
+  ActMask m{};
+  for (size_t t = 0; t < v.size() && t < (size_t)kMaxR; t++)
+    if (v[t]) m.w[t >> 5] |= 1u << (t & 31);
+  launch_set_act(act.as<int>() + slot * kMaxR, m, stream);
+}
+
+// r.r, b.x and x.r of the last residual launch (np partials each), one wait
+void Context::read_residual(double *rr, double *bx, double *xr, int np) {
+  launch_finalize3(red, S_RR, S_BX, S_XR, R, np, stream);
+  FEMH_HIP(hipGetLastError());
+  double h[3 * kMaxR];
+  FEMH_HIP(hipMemcpyAsync(h, red.scalars + S_RR * kSlotWidth, sizeof(h), hipMemcpyDeviceToHost, stream));
   FEMH_HIP(hipStreamSynchronize(stream));
+  std::copy(h, h + R, rr);
+  std::copy(h + kMaxR, h + kMaxR + R, bx);
+  std::copy(h + 2 * kMaxR, h + 2 * kMaxR + R, xr);
 }
 
 void Context::read_scalars(int slot, double *out, int n, int np) {
@@ -358,7 +368,6 @@ void Context::build_levels(Hierarchy<T> &h) {
     L.g = dims[l];
     L.D.alloc(sizeof(T) * 3 * B * L.g.V);
     L.Dinv.alloc(sizeof(T) * 3 * B * L.g.V);
-    L.lmax.assign(B, 0.0);
     // V-cycle work vectors (a one-level hierarchy -- Jacobi -- needs none;
     // the autotuner and apply_level take theirs on first use)
     if (dims.size() > 1)
@@ -383,12 +392,15 @@ void Context::estimate_lmax(Hierarchy<T> &h) {
   for (int s = 0; s < nb; s++) pw[kRHS * s] = 1;
   set_act(A_POW, pw);
   const int *ap = actp(A_POW);
+  if (h.lv.size() > (size_t)kMaxLevels) throw Error(FEMH_DEVICE_ERROR, "too many levels");
+  lm_part.alloc(sizeof(double) * h.lv.size() * 2 * kMaxB * kRedBlocks);
+  lmax_d.alloc(sizeof(double) * kMaxLevels * kMaxB);
   for (size_t l = 0; l < h.lv.size(); l++) {
     Level<T> &L = h.lv[l];
     const int V = L.g.V;
     T *xv = L.x.template as<T>(), *yv = L.Ad.template as<T>();
     // every sample starts from the same vector (batched == one-sample results)
-    launch_fill_hash<T>((size_t)R * 3 * V, (size_t)kRHS * 3 * V, xv, 0x51ED27ull + l, stream);
+    launch_fill_hash<T>((size_t)3 * V, (size_t)kRHS * 3 * V, nb, xv, 0x51ED27ull + l, stream);
     // y_k = (D^-1 A)^k x_0 without normalising (ten steps grow it by at most
     // lambda^10 <= 1e10 or so), one fused launch per step; the estimate
     // ||y_10|| / ||y_9|| is that of the normalised iteration.  It approaches
@@ -414,18 +426,53 @@ void Context::estimate_lmax(Hierarchy<T> &h) {
       op<T>(h, (int)l, ST_PLAIN, EP_AXD, a);
       std::swap(xv, yv);
     }
-    launch_dot<T>(V, R, yv, yv, S_AUX, ap, red, stream);  // y_9
-    launch_dot<T>(V, R, xv, xv, S_RR, ap, red, stream);   // y_10
+    launch_power_norms<T>(V, nb, (int)l, yv, xv, lm_part.as<double>(), stream);  // y_9, y_10
     FEMH_HIP(hipGetLastError());
-    std::vector<double> n9(R), n10(R);
-    read_scalars(S_AUX, n9.data(), R, vec_parts(V));
-    read_scalars(S_RR, n10.data(), R, vec_parts(V));
-    for (int s = 0; s < nb; s++) {
-      const double a9 = n9[kRHS * s], a10 = n10[kRHS * s];
-      L.lmax[s] = kLmaxScale * std::sqrt(a9 > 0 ? std::max(a10, 0.0) / a9 : 0.0);
-      if (!(L.lmax[s] > 0) || !std::isfinite(L.lmax[s]))
-        throw Error(FEMH_NONFINITE, "operator is not finite");
-    }
+  }
+  cheb_setup(h, true);
+}
+
+// lambda_max of every level and sample (with norms; else those that lmax_d
+// holds) and the device table of Chebyshev coefficients of h that follows
+template <typename T>
+void Context::cheb_setup(Hierarchy<T> &h, bool norms) {
+  const int L = (int)h.lv.size();
+  ChebSetup cs{};
+  for (int l = 0; l < L; l++) cs.np[l] = vec_parts(h.lv[l].g.V);
+  cs.steps = std::max(kMaxCheb, std::max(2, o.coarse_iters)) + 1;
+  cs.ratio[0] = o.cheby_ratio;
+  cs.ratio[1] = kCoarseChebRatio;
+  cs.scale = kLmaxScale;
+  h.cheb.alloc(sizeof(double) * (size_t)L * cs.steps * 2 * 3 * kMaxB);
+  launch_cheb_setup(L, nb, cs, norms ? lm_part.as<double>() : nullptr, lmax_d.as<double>(), h.cheb.template as<double>(),
+                    stream);
+  FEMH_HIP(hipGetLastError());
+  h.cheb_steps = cs.steps;
+}
+
+// Raises what the set-up kernels found (spectrum estimates that are not finite,
+// a coarsest operator that is not positive definite).  Their flags come with
+// the scalars of slots S_BB and S_AUX (out: 2 kSlotWidth doubles, may be null),
+// so that the host waits once for the whole set-up.
+void Context::check_setup(double *out) {
+  const bool mg = o.precond == FEMH_PRECOND_MG && nlevels > 1;
+  static_assert(S_AUX == S_BB + 1 && kMaxR + kMaxB <= kSlotWidth, "the report follows the b.b values");
+  if (mg)
+    launch_setup_report(nb, nlevels, lmax_d.as<double>(), ndense_of() ? dense_bad.as<int>() : nullptr,
+                        red.scalars + S_BB * kSlotWidth + kMaxR, stream);
+  FEMH_HIP(hipGetLastError());
+  std::vector<double> h(2 * kSlotWidth);
+  FEMH_HIP(hipMemcpyAsync(h.data(), red.scalars + S_BB * kSlotWidth, sizeof(double) * h.size(),
+                          hipMemcpyDeviceToHost, stream));
+  FEMH_HIP(hipStreamSynchronize(stream));
+  if (out) std::copy(h.begin(), h.end(), out);
+  else if (mg) raise_setup(h.data());
+}
+
+void Context::raise_setup(const double *scalars) const {
+  for (int s = 0; s < nb; s++) {
+    if (scalars[kMaxR + s] == 1.0) throw Error(FEMH_NONFINITE, "operator is not finite");
+    if (scalars[kMaxR + s] == 2.0) throw Error(FEMH_NONFINITE, "coarsest operator is not positive definite");
   }
 }
 
@@ -445,11 +492,6 @@ void Context::dense_coarse(Hierarchy<T> &h) {
   launch_dense_inverse<T>(L.g, nb, L.S.template as<T>(), dense_work.as<double>(), h.Ainv.template as<T>(),
                           dense_bad.as<int>(), stream);
   FEMH_HIP(hipGetLastError());
-  int bad[kMaxB];
-  FEMH_HIP(hipMemcpyAsync(bad, dense_bad.p, sizeof(int) * nb, hipMemcpyDeviceToHost, stream));
-  FEMH_HIP(hipStreamSynchronize(stream));
-  for (int smp = 0; smp < nb; smp++)
-    if (bad[smp]) throw Error(FEMH_NONFINITE, "coarsest operator is not positive definite");
   h.ndense = n;
 }
 
@@ -529,7 +571,7 @@ void Context::autotune(Hierarchy<T> &h) {
     Level<T> &Lv = h.lv[l];
     Lv.d.alloc(field_bytes(Lv.g, B, sizeof(T)));
     Lv.Ad.alloc(field_bytes(Lv.g, B, sizeof(T)));
-    launch_fill_hash<T>((size_t)R * 3 * Lv.g.V, (size_t)kRHS * 3 * Lv.g.V, Lv.d.template as<T>(), 0x7A11ull + l,
+    launch_fill_hash<T>((size_t)kRHS * 3 * Lv.g.V, (size_t)kRHS * 3 * Lv.g.V, nb, Lv.d.template as<T>(), 0x7A11ull + l,
                         stream);
   }
   FEMH_HIP(hipGetLastError());
@@ -596,7 +638,6 @@ void Context::build_hierarchy() {
     // (a grid with an odd edge has one level: Jacobi, no smoother)
     if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
       estimate_lmax(h64);
-      upload_cheb(h64);
       // the coarsest level is inverted densely when it is small enough, else
       // solved approximately by a long Chebyshev polynomial (cheb_run)
       dense_coarse(h64);
@@ -612,8 +653,6 @@ void Context::build_hierarchy() {
     if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
       dense_coarse(h32);
       estimate_lmax(h32);
-      upload_cheb(h32);
-      for (int l = 0; l < nlevels; l++) h64.lv[l].lmax = h32.lv[l].lmax;
     }
     FEMH_HIP(hipGetLastError());
     h32.ready = true;
@@ -627,57 +666,14 @@ void Context::ensure_h64_ops() {
   // (spectrum bounds stay those of the FP32 operators)
   if (o.precond == FEMH_PRECOND_MG && nlevels > 1) {
     dense_coarse(h64);
-    upload_cheb(h64);
+    cheb_setup(h64, false);
+    check_setup();
   }
   h64_ops = true;
 }
 
 // ---------------------------------------------------------------------------
 // multigrid V-cycle with Chebyshev smoothing (fused kernels, see ops.hpp)
-// Chebyshev iteration for D^-1 A on [lmax/ratio, lmax]: 1/theta and the
-// coefficients (c1, c2) of step `step` (1-based) of the three-term recurrence
-// d_s = c1 d_{s-1} + c2 D^-1 r_s.
-static void cheb_step(double lmax, double ratio, int step, double *theta_inv, double *c1, double *c2) {
-  const double hi = lmax, lo = lmax / ratio;
-  const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
-  *theta_inv = 1.0 / theta;
-  double rho = 1.0 / sigma;
-  *c1 = *c2 = 0.0;
-  for (int s = 1; s <= step; s++) {
-    const double rn = 1.0 / (2.0 * sigma - rho);
-    *c1 = rn * rho;
-    *c2 = 2.0 * rn / delta;
-    rho = rn;
-  }
-}
-
-// the device table of Chebyshev coefficients of h (after its spectrum
-// estimates): per level, step and interval, 1/theta and (from step 1 on) c1
-// and c2 of every sample
-template <typename T>
-void Context::upload_cheb(Hierarchy<T> &h) {
-  const int L = (int)h.lv.size();
-  const int steps = std::max(kMaxCheb, std::max(2, o.coarse_iters)) + 1;
-  const size_t per = (size_t)3 * kMaxB;
-  std::vector<double> tab((size_t)L * steps * 2 * per, 0.0);
-  for (int l = 0; l < L; l++)
-    for (int st = 0; st < steps; st++)
-      for (int kind = 0; kind < 2; kind++) {
-        double *t = tab.data() + (((size_t)l * steps + st) * 2 + kind) * per;
-        for (int s = 0; s < nb; s++) {
-          double ti, c1, c2;
-          cheb_step(h.lv[l].lmax[s], kind ? kCoarseChebRatio : o.cheby_ratio, st, &ti, &c1, &c2);
-          t[s] = ti;
-          t[kMaxB + s] = st >= 1 ? c1 : 0.0;
-          t[2 * kMaxB + s] = st >= 1 ? c2 : 0.0;
-        }
-      }
-  h.cheb.alloc(sizeof(double) * tab.size());
-  FEMH_HIP(hipMemcpyAsync(h.cheb.p, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice, stream));
-  FEMH_HIP(hipStreamSynchronize(stream));
-  h.cheb_steps = steps;
-}
-
 // per-sample 1/theta and the coefficients of Chebyshev step `step` (1-based):
 // the launch reads them from the hierarchy's device table
 template <typename T>
@@ -934,13 +930,16 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     else
       launch_p_update<T>(V, R, pv, zv, rzn, rzc, 0, ap, red, np_rz, stream, lz_beta, cnt);
   };
-  std::vector<int> hact(kMaxR), hst(kMaxR);
   int nlive = nact;
   // host look at the device state: false when no right-hand side is left.
   // Only k_pcg_check clears a right-hand side's activity, and it sets the
   // state (1 or 2) when it does, so the state alone tells which are left.
+  // (one copy: iteration counts and states, then relative residuals)
+  std::vector<double> hstate(2 * kMaxR);
+  const int *hcnt = reinterpret_cast<const int *>(hstate.data()), *hst = hcnt + kMaxR;
+  const double *hrel = hstate.data() + kMaxR;
   auto poll = [&]() {
-    FEMH_HIP(hipMemcpyAsync(hst.data(), pst, sizeof(int) * R, hipMemcpyDeviceToHost, stream));
+    FEMH_HIP(hipMemcpyAsync(hstate.data(), pcg_state.p, sizeof(double) * hstate.size(), hipMemcpyDeviceToHost, stream));
     FEMH_HIP(hipStreamSynchronize(stream));
     nlive = 0;
     for (int t = 0; t < R; t++) {
@@ -1037,20 +1036,14 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     const int every = jac ? std::max(o.check_every, std::min(8, it / 8)) : o.check_every;
     if (it % std::max(every, 1) == 0 || it == max_iter) live = poll();
   }
-  if (live) poll();
-  // results of the run: iterations and residual per right-hand side, and the
-  // activity that remains (not converged within max_iter)
-  std::vector<int> hcnt(R);
-  std::vector<double> hrel(R);
-  FEMH_HIP(hipMemcpyAsync(hcnt.data(), cnt, sizeof(int) * R, hipMemcpyDeviceToHost, stream));
-  FEMH_HIP(hipMemcpyAsync(hrel.data(), relres_d, sizeof(double) * R, hipMemcpyDeviceToHost, stream));
-  FEMH_HIP(hipMemcpyAsync(hact.data(), apw, sizeof(int) * R, hipMemcpyDeviceToHost, stream));
-  FEMH_HIP(hipStreamSynchronize(stream));
+  // results of the run: iterations and residual per right-hand side, and which
+  // are left (not converged within max_iter)
+  if (live || max_iter == 1) poll();
   for (int t = 0; t < R; t++) {
     if (!active[t]) continue;
     iters[t] = hcnt[t];
     relres[t] = hrel[t];
-    active[t] = hact[t] != 0;
+    active[t] = hst[t] == 0;
   }
   FEMH_HIP(hipGetLastError());
 }
@@ -1175,7 +1168,8 @@ void Context::homogenize(double *C, femh_stats *st) {
   const bool timed = ev[0] != nullptr;
   if (timed) FEMH_HIP(hipEventRecord(ev[0], stream));
   have_fields = false;
-  // validate the moduli before any device work depends on them
+  // The moduli are checked with the set-up's other results, in one wait at its
+  // end: no kernel's indexing or trip count depends on their values.
   // cubic structure: a cell takes the two-solve path only if its moduli are
   // invariant under the axis swaps (counted on the device); other cells of
   // the batch are solved with all six load cases
@@ -1184,14 +1178,7 @@ void Context::homogenize(double *C, femh_stats *st) {
   std::vector<char> cubic_ok(nb, 0);
   {
     const int np = launch_modulus_stats(g.V, nb, E64.as<double>(), red, stream, cubic ? g.nx : 0);
-    read_scalars(S_AUX, mst.data(), (cubic ? 4 : 3) * nb, np);
-    if (cubic)
-      for (int s = 0; s < nb; s++) cubic_ok[s] = mst[3 * nb + s] == 0.0;
-  }
-  for (int s = 0; s < nb; s++) {
-    if (mst[3 * s + 1] > 0) throw Error(FEMH_NONFINITE, "non-finite modulus");
-    if (mst[3 * s + 2] > 0) throw Error(FEMH_BAD_ARG, "negative modulus");
-    if (!(mst[3 * s] > 0)) throw Error(FEMH_BAD_ARG, "all-void cell (every modulus is zero)");
+    launch_finalize(red, S_AUX, (cubic ? 4 : 3) * nb, np, stream);
   }
   std::vector<int> all(R, 1);
   set_act(A_ALL, all);
@@ -1202,9 +1189,19 @@ void Context::homogenize(double *C, femh_stats *st) {
   const bool cold_mixed = o.precision == FEMH_MIXED && !warm;
   launch_fine_rhs<double>(f0, R, gtab.as<double>(), b.as<double>(), cold_mixed ? r32.as<float>() : nullptr,
                           red, S_BB, stream);
-  FEMH_HIP(hipGetLastError());
-  std::vector<double> bb(R);
-  read_scalars(S_BB, bb.data(), R, vec_parts(g.V));
+  launch_finalize(red, S_BB, R, vec_parts(g.V), stream);
+  std::vector<double> setup(2 * kSlotWidth);
+  check_setup(setup.data());
+  std::copy(setup.begin() + kSlotWidth, setup.begin() + kSlotWidth + mst.size(), mst.begin());
+  for (int s = 0; s < nb; s++) {
+    if (mst[3 * s + 1] > 0) throw Error(FEMH_NONFINITE, "non-finite modulus");
+    if (mst[3 * s + 2] > 0) throw Error(FEMH_BAD_ARG, "negative modulus");
+    if (!(mst[3 * s] > 0)) throw Error(FEMH_BAD_ARG, "all-void cell (every modulus is zero)");
+  }
+  if (o.precond == FEMH_PRECOND_MG && nlevels > 1) raise_setup(setup.data());
+  if (cubic)
+    for (int s = 0; s < nb; s++) cubic_ok[s] = mst[3 * nb + s] == 0.0;
+  std::vector<double> bb(setup.begin(), setup.begin() + R);
   // right-hand sides that vanish (the affine field already balances, e.g. a
   // homogeneous cell) are solved by u = 0
   std::vector<int> active(R, 0);
@@ -1273,9 +1270,7 @@ void Context::homogenize(double *C, femh_stats *st) {
     std::vector<double> bx(R, 0.0), xr(R, 0.0), rz(R), rn(R), bxn(R), xrn(R);
     if (warm) {
       const int npd = residual_dots(actp(A_ALL));
-      read_scalars(S_RR, rr.data(), R, npd);
-      read_scalars(S_BX, bx.data(), R, npd);
-      read_scalars(S_XR, xr.data(), R, npd);
+      read_residual(rr.data(), bx.data(), xr.data(), npd);
       for (int t = 0; t < R; t++)
         if (active[t]) {
           relres[t] = std::sqrt(rr[t] / bb[t]);
@@ -1430,9 +1425,7 @@ void Context::homogenize(double *C, femh_stats *st) {
       }
       const int npd = residual_dots(ao);
       FEMH_HIP(hipGetLastError());
-      read_scalars(S_RR, rn.data(), R, npd);
-      read_scalars(S_BX, bxn.data(), R, npd);
-      read_scalars(S_XR, xrn.data(), R, npd);
+      read_residual(rn.data(), bxn.data(), xrn.data(), npd);
       // A sweep that did not reach its tolerance, or that failed to halve the
       // FP64 residual, means the FP32 hierarchy does not precondition this
       // cell (FP32 rounding of operators with a modulus contrast near its

@@ -85,7 +85,6 @@ struct Level {
   Dims g{};
   DBuf S;                    // stencil [B][243][V] (levels >= 1)
   DBuf D, Dinv;              // point diagonal and its inverse [B][3][V]
-  std::vector<double> lmax;  // per sample: lambda_max(D^-1 A) estimate (with margin)
   DBuf x, b, r, d, d2, xn, Ad;  // V-cycle work, [R][3][V]
 };
 
@@ -155,6 +154,9 @@ struct Context {
   // PCG iteration state on the device: iterations, state (int [kMaxR] each),
   // relative residual and |b|^2 (double [kMaxR] each)
   DBuf pcg_state;
+  // power iteration: norm partials [kMaxLevels][2][kMaxB][kRedBlocks]; lambda_max
+  // (with margin) of every level and sample [kMaxLevels][kMaxB]
+  DBuf lm_part, lmax_d;
   DBuf dense_work, dense_bad;  // dense coarsest inverse: FP64 matrices and panels, per-sample failure flag
   DBuf ls_part, ls_h;  // device line search: per-cell block partials [n][kRedBlocks], steps [n]
   // recorded PCG iteration pairs (hipGraph), keyed by everything their
@@ -220,6 +222,7 @@ struct Context {
   // inputs: n samples (<= B) of density (interp applied) or modulus
   void load(const double *src, int n, bool device_src, bool modulus);
   void build_hierarchy();
+  void check_setup(double *out = nullptr);
   // FP64 level operators of a mixed-precision context, built on first use
   // (the FP64 fallback, apply_level); mixed solves smooth with FP32 ones
   void ensure_h64_ops();
@@ -276,7 +279,9 @@ struct Context {
   template <typename T>
   void set_cheb(const Hierarchy<T> &h, int l, OpArgs<T> &a, int step, double ratio);
   template <typename T>
-  void upload_cheb(Hierarchy<T> &h);
+  void cheb_setup(Hierarchy<T> &h, bool norms);
+  void raise_setup(const double *scalars) const;
+  int ndense_of() const { return o.precision == FEMH_MIXED && !h64_ops ? h32.ndense : h64.ndense; }
   template <typename T>
   void cheb_run(Hierarchy<T> &h, int l, const T *b, T *x, const int *act_, int k, double ratio);
   int apply_parts(int sz) const;  // partials of a fine-operator dot, element size sz
@@ -289,6 +294,7 @@ struct Context {
   template <typename T>
   void dense_coarse(Hierarchy<T> &h);
   void read_scalars(int slot, double *out, int n, int np);
+  void read_residual(double *rr, double *bx, double *xr, int np);
   void compute_ch(const double *fields, double *C);
 };
 
