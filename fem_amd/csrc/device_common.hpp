@@ -72,6 +72,22 @@ static __device__ __forceinline__ double sum_parts(const Reduce &red, int slot, 
   return block_sum(s);
 }
 
+// The same value, bit for bit, without a barrier: every wave sums what the four
+// waves of a 256-thread block would, and every lane receives it (any block
+// size; for kernels that need the scalar before they start on their data).
+static __device__ __forceinline__ double sum_parts_wave(const Reduce &red, int slot, int idx, int np) {
+  const double *pp = red.partials + ((size_t)slot * kSlotWidth + idx) * kMaxPartials;
+  double t[kBlock / 64];
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; w++) {
+    t[w] = 0;
+    if (np <= 64 * w) continue;
+    for (int i = 64 * w + (threadIdx.x & 63); i < np; i += kBlock) t[w] += pp[i];
+    t[w] = wave_sum(t[w]);
+  }
+  return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 static inline int grid_for(int V) {
   int b = (V + kBlock - 1) / kBlock;
   return b < kRedBlocks ? (b < 1 ? 1 : b) : kRedBlocks;

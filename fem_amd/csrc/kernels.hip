@@ -510,6 +510,17 @@ __global__ __launch_bounds__(kBlock) void k_beta(int rz_new, int rz_old, int fir
   }
 }
 
+__global__ __launch_bounds__(kBlock) void k_x_last(int V, float *__restrict__ x, const float *__restrict__ p0,
+                                                   const float *__restrict__ p1, const double *__restrict__ alpha,
+                                                   const int *__restrict__ cnt) {
+  const int rr = blockIdx.y, k = cnt[rr];
+  if (k <= 0) return;
+  const float a = (float)alpha[rr];
+  const size_t off = (size_t)rr * 3 * V;
+  const float *__restrict__ p = (k & 1) ? p1 : p0;
+  for (int t = blockIdx.x * kBlock + threadIdx.x; t < 3 * V; t += gridDim.x * kBlock) x[off + t] += a * p[off + t];
+}
+
 // PCG convergence test on the device, one block per right-hand side: the
 // residual norm from the S_RR partials gives relres = sqrt(r.r / b.b); a
 // right-hand side that reaches tol (state 1) or turns non-finite (state 2)
@@ -1160,6 +1171,10 @@ void launch_p_update(int V, int R, T *p, const T *z, int rz_new, int rz_old, int
                      const int *cnt) {
   hipLaunchKernelGGL(k_p_update<T>, grid2(3 * V, R), dim3(kBlock), 0, s, V, p, z, rz_new, rz_old,
                      first, act, red, np_rz, beta_out, cnt);
+}
+void launch_x_last(int V, int R, float *x, const float *p0, const float *p1, const double *alpha, const int *cnt,
+                   hipStream_t s) {
+  hipLaunchKernelGGL(k_x_last, grid2(3 * V, R), dim3(kBlock), 0, s, V, x, p0, p1, alpha, cnt);
 }
 void launch_pcg_check(int R, int *act, const Reduce &red, int np, const double *bb, double tol, int *cnt,
                       double *relres, int *state, hipStream_t s, int rz_new, int rz_old, double *beta,

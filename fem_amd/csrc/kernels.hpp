@@ -185,6 +185,10 @@ void launch_p_update(int V, int R, T *p, const T *z, int rz_new, int rz_old, int
 // direction update of the fine operator (ST_PUPD); beta_out as for p_update
 void launch_beta(int R, int rz_new, int rz_old, int first, const int *act, const Reduce &red, int np_rz,
                  double *beta, hipStream_t s, double *beta_out = nullptr, const int *cnt = nullptr);
+// x += alpha p of the last iteration of every RHS that did one (cnt > 0): p1
+// after an odd number of iterations, p0 after an even one
+void launch_x_last(int V, int R, float *x, const float *p0, const float *p1, const double *alpha, const int *cnt,
+                   hipStream_t s);
 // PCG convergence check on the device (after the update of an iteration):
 // for every active RHS, cnt += 1 and relres = sqrt(r.r / bb) from the np
 // partials of S_RR; relres <= tol clears act (state 1), a non-finite r.r too

@@ -49,7 +49,8 @@ __device__ __forceinline__ int wrap1(int i, int n) { return i < 0 ? i + n : (i >
 // load behind a run-time branch is waited for at the branch's end):
 //   EP_RES, EP_PRE: e0 = b ; EP_CHEB0, EP_CHEB0L, EP_FIN1: e0 = b, e1 = 1/D ;
 //   EP_STEP, EP_LAST, EP_LASTD: e0 = rprev, e1 = 1/D, e2 = xprev (none from a
-//   zero start, ST_DSCALE) ; EP_LASTD: e3 = b (for b . x) ; EP_AXD: e1 = 1/D
+//   zero start, ST_DSCALE) ; EP_LASTD: e3 = b (for b . x) ; EP_AXD: e1 = 1/D ;
+//   ST_PUPDX: e1 = the old direction, e2 = x
 template <typename T>
 struct EpiIn {
   T e0[3], e1[3], e2[3], e3[3];
@@ -70,6 +71,10 @@ __device__ __forceinline__ void epi_load(const OpArgs<T> &a, const T *__restrict
     if (EP == EP_CHEB0 || EP == EP_FIN1 || ep_is_step(EP) || EP == EP_AXD) p.e1[c] = Ds[(size_t)c * V + n];
     if (ep_is_step(EP)) p.e2[c] = ST == ST_DSCALE ? (T)0 : a.xprev[q];
     if (EP == EP_LASTD) p.e3[c] = a.b[q];
+    if (ST == ST_PUPDX) {
+      p.e1[c] = a.u2[q];
+      p.e2[c] = a.x[q];
+    }
   }
 }
 
@@ -94,13 +99,14 @@ __device__ __forceinline__ void ep_store(T *p, T v) {
 template <typename T, int ST, int EP, bool NT = false>
 __device__ __forceinline__ void epilogue(const OpArgs<T> &a, const EpiIn<T> &p, T ti, T c1, T c2,
                                          size_t off, int V, int n, const T Au[3], const T uo[3],
-                                         DotAcc &dv) {
+                                         DotAcc &dv, T al = 0) {
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     const size_t q = off + (size_t)c * V + n;
     if (EP == EP_AX) {
       ep_store<NT>(&a.y[q], Au[c]);
-      if (ST == ST_PUPD) ep_store<NT>(&a.pout[q], uo[c]);
+      if (ST == ST_PUPD || ST == ST_PUPDX) ep_store<NT>(&a.pout[q], uo[c]);
+      if (ST == ST_PUPDX) ep_store<NT>(&a.x[q], p.e2[c] + al * p.e1[c]);
       if (a.dot) dv.a += (double)uo[c] * (double)Au[c];
     } else if (EP == EP_AXD) {
       ep_store<NT>(&a.y[q], Au[c] * p.e1[c]);
@@ -327,14 +333,19 @@ __device__ __forceinline__ double bload(__amdgpu_buffer_rsrc_t r, unsigned voff,
 //    is then never stored).  The coarse nodes around the tile are staged into
 //    cl one coarse plane at a time, two slabs ahead; each staging slot keeps
 //    its interpolated value of the lower coarse plane.
-// Waves per SIMD the FP32 variants are compiled for: 4 (at most 128 VGPRs).
-template <typename T>
+//  * Residual update (RUPD): r' = r - alpha q is formed where it is staged,
+//    (theta D)^-1 r' goes to the staged plane and r' itself to rb, whose three
+//    planes rotate: one being staged, one turned into the residual in place, one
+//    being restricted.
+// Waves per SIMD the FP32 variants are compiled for: 4 (at most 128 VGPRs);
+// three where the 256-thread tiles' LDS lets no fourth workgroup in (RUPD).
+template <typename T, int ST, int NT>
 constexpr int tiled_waves() {
-  return sizeof(T) == 4 ? 4 : kWaves64;
+  return sizeof(T) != 4 ? kWaves64 : ST == ST_RUPD && NT < 512 ? 3 : 4;
 }
 
 template <typename T, int ST, int EP, int TJ, int TK, bool RS>
-__global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, const T *__restrict__ E,
+__global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, TJ * TK>())) void k_tiled(Dims g, const T *__restrict__ E,
                                                                            ModeC<T> mc, OpArgs<T> a, int TI,
                                                                            int tiles_k, int tiles, int chunks) {
   constexpr int NT = TJ * TK;                           // threads = owned nodes per plane
@@ -344,7 +355,9 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   constexpr int QS = (NS + NT - 1) / NT, QE = (NE + NT - 1) / NT;
   static_assert(NT % 64 == 0 && QS <= 2 && QE <= 2, "tile shape");
   constexpr bool kProl = ST == ST_PROLONG || ST == ST_DPROLONG;
-  constexpr bool kStD = ST == ST_DSCALE || ST == ST_DPROLONG;  // stages b / (theta D)
+  constexpr bool kStD = ST == ST_DSCALE || ST == ST_DPROLONG || ST == ST_RUPD;  // stages b / (theta D)
+  constexpr bool kPupd = ST == ST_PUPD || ST == ST_PUPDX, kRupd = ST == ST_RUPD;
+  static_assert(!kRupd || RS, "the residual update stages for the restricted residual");
   constexpr int CJ = TJ / 2 + 2, CK = TK / 2 + 2;              // coarse nodes around the tile (kProl)
   constexpr unsigned SZ = sizeof(T);
   const int inner = EP == EP_AXD ? 1 : kRHS;  // (the power iteration runs load case 0 only)
@@ -358,15 +371,27 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   const T *__restrict__ Ds = a.Dinv ? a.Dinv + (size_t)smp * 3 * V : nullptr;
   const size_t off = (size_t)r * 3 * V;
   const __amdgpu_buffer_rsrc_t rU = brsrc(a.u + off, 3 * VB);
-  const __amdgpu_buffer_rsrc_t rU2 = brsrc(ST == ST_PUPD ? a.u2 + off : a.u + off, 3 * VB);
+  const __amdgpu_buffer_rsrc_t rU2 = brsrc(kPupd || kRupd ? a.u2 + off : a.u + off, 3 * VB);
   const __amdgpu_buffer_rsrc_t rD = brsrc(Ds ? Ds : a.u + off, 3 * VB);
   const T ti = a.cheb ? (T)a.cheb[smp] : (T)0, c1 = a.cheb ? (T)a.cheb[kMaxB + smp] : (T)0,
           c2 = a.cheb ? (T)a.cheb[2 * kMaxB + smp] : (T)0;
-  const T bt = ST == ST_PUPD ? (T)a.beta[r] : (T)0;
+  T bt = ST == ST_PUPD ? (T)a.beta[r] : (T)0, al = ST == ST_PUPDX ? (T)a.alpha[r] : (T)0;
+  if constexpr (ST == ST_PUPDX || kRupd) {
+    const double num = sum_parts_wave(a.red, a.slot2, r, a.np), den = sum_parts_wave(a.red, a.slot3, r, a.np3);
+    const double v = den != 0.0 ? num / den : 0.0;
+    (kRupd ? al : bt) = (T)v;
+    if (id.unit == 0 && threadIdx.x == 0) {
+      if (kRupd) a.alpha[r] = v;
+      if (a.record) a.record[(size_t)(a.cnt[r] - (kRupd ? 0 : 1)) * kMaxR + r] = v;
+    }
+  }
   __shared__ T up[2][3 * NS];
   __shared__ T eo[NE * kEOH];
   __shared__ T cl[kProl ? 3 * CJ * CK : 1];
-  __shared__ T rb[RS ? 3 * (TJ + 1) * (TK + 1) : 1];
+  // (kRupd: plane ip's r' waits in part (ip - i0) mod 3 from its staging until the
+  // gather turns it into the residual in place, and that until its restriction)
+  constexpr int RP = 3 * (TJ + 1) * (TK + 1);
+  __shared__ T rb[RS ? (kRupd ? 3 : 1) * RP : 1];
   const int tid = threadIdx.x;
   // staging slots and voxels go to threads in an order rotated by a wave per
   // workgroup, so that the second round of the extra ones does not fall on
@@ -463,7 +488,7 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   // staging of node plane ip into LDS buffer buf, software-pipelined: fetch()
   // issues the loads of a plane into registers one slab ahead, put() scales
   // and stores them.
-  T pf[QS][3], pd[QS][3];
+  T pf[QS][3], pd[QS][3], pq[kRupd ? QS : 1][3];
   auto fetch = [&](int ip) {
     const int iw = wrap1(ip, g.nx);
 #pragma unroll
@@ -474,19 +499,35 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
       for (int c = 0; c < 3; c++) {
         pf[q][c] = bload(rU, vo, c * VB, (T *)nullptr);
         if (kStD) pd[q][c] = bload(rD, vo, c * VB, (T *)nullptr);
-        if (ST == ST_PUPD) pd[q][c] = bload(rU2, vo, c * VB, (T *)nullptr);
+        if (kPupd) pd[q][c] = bload(rU2, vo, c * VB, (T *)nullptr);
+        if constexpr (kRupd) pq[q][c] = bload(rU2, vo, c * VB, (T *)nullptr);
       }
     }
   };
+  int part = 0;  // kRupd: offset in rb of the plane the slab completes
   auto put = [&](int buf, int ip) {
 #pragma unroll
     for (int q = 0; q < QS; q++) {
       if (soff[q] < 0) continue;
       T *dst = &up[buf][3 * (vt + q * NT)];
       T v[3];
+      if constexpr (kRupd) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) pf[q][c] = pf[q][c] - al * pq[q][c];
+        // place of the staged node among the owned and extra ones, derived anew
+        // (not kept over the loop; see cpk)
+        int t = vt + q * NT;
+        asm volatile("" : "+v"(t));
+        const int sj = t / NK - 1, sk = t - (sj + 1) * NK - 1;
+        if (sj >= 0 && sj <= TJ && sk >= 0 && sk <= TK) {
+          T *up1 = rb + (part == 2 * RP ? 0 : part + RP);
+#pragma unroll
+          for (int c = 0; c < 3; c++) up1[(c * (TJ + 1) + sj) * (TK + 1) + sk] = pf[q][c];
+        }
+      }
 #pragma unroll
       for (int c = 0; c < 3; c++)
-        v[c] = kStD ? pf[q][c] * (ti * pd[q][c]) : (ST == ST_PUPD) ? pf[q][c] + bt * pd[q][c] : pf[q][c];
+        v[c] = kStD ? pf[q][c] * (ti * pd[q][c]) : kPupd ? pf[q][c] + bt * pd[q][c] : pf[q][c];
       if constexpr (kProl) {
         // (x is rounded before the correction is added, as when it is stored)
 #pragma clang fp contract(off)
@@ -528,11 +569,11 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   double racc = 0;  // RS: this thread's coarse node sum
   // RS: restriction of residual plane ip in rb: rows and columns with weights
   // 1/2, 1, 1/2, planes 2I - 1, 2I, 2I + 1 into coarse plane I
-  auto restrict_plane = [&](int ip) {
+  auto restrict_plane = [&](int ip, int at) {
     constexpr int CN = (TJ / 2) * (TK / 2);
     if (tid >= 3 * CN) return;
     const int c = tid / CN, q = tid - c * CN, J = q / (TK / 2), K = q - J * (TK / 2);
-    const T *p = rb + c * (TJ + 1) * (TK + 1) + 2 * J * (TK + 1) + 2 * K;
+    const T *p = rb + at + c * (TJ + 1) * (TK + 1) + 2 * J * (TK + 1) + 2 * K;
     double s = 0;
 #pragma unroll
     for (int oj = 0; oj < 3; oj++) {
@@ -631,7 +672,7 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
   fetch(i0 - 1 - H);
   put(0, i0 - 1 - H);
   fetch(i0 - H);
-  for (int sl = i0 - 1 - H, p = 0; sl < iend; sl++, p++) {
+  for (int sl = i0 - 1 - H, p = 0; sl < iend; sl++, p++, part = !kRupd ? 0 : part == 2 * RP ? 0 : part + RP) {
     const int cur = p & 1, nxt = cur ^ 1;
     const int sw = wrap1(sl, g.nx);
     // loads in the order they are consumed: moduli of this slab, epilogue
@@ -642,9 +683,10 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
       Ev[q] = eoff[q] >= 0 ? bload(rE, (unsigned)(sw * plane + eoff[q]) * SZ, 0u, (T *)nullptr) : (T)0;
     const size_t nown = (size_t)sw * plane + gj * g.nz + gk;
     EpiIn<T> pin;
-    if (EP != EP_AX && p > 0 && owns) epi_load<T, ST, EP>(a, Ds, off, V, (int)nown, pin);
+    if ((EP != EP_AX || ST == ST_PUPDX) && !kRupd && p > 0 && owns)
+      epi_load<T, ST, EP>(a, Ds, off, V, (int)nown, pin);
     T xin[3];
-    if constexpr (RS) {
+    if constexpr (RS && !kRupd) {
       if (p > 0 && extra) {
 #pragma unroll
         for (int c = 0; c < 3; c++)
@@ -657,13 +699,26 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
     // slab; the previous slab's gather of eo is behind that barrier too)
     __syncthreads();
     if constexpr (RS) {
-      if (p > 1) restrict_plane(sl - 1);
+      if (p > 1) restrict_plane(sl - 1, !kRupd ? 0 : part == 0 ? 2 * RP : part - RP);
     }
     if constexpr (kProl) {
       // (the odd plane that reads cl is put in the next slab)
       if (!(p & 1)) {
         cput();
         cfetch((sl + 1) / 2 + 2);
+      }
+    }
+    if constexpr (kRupd) {
+      if (p > 0 && sl >= i0 && owns) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          const T v = rb[part + (c * (TJ + 1) + nj + 1) * (TK + 1) + nk + 1];
+          if (a.nt)
+            ep_store<true>(&a.pout[off + (size_t)c * V + nown], v);
+          else
+            ep_store<false>(&a.pout[off + (size_t)c * V + nown], v);
+          dv.a += (double)v * (double)v;
+        }
       }
     }
     T uo[3];
@@ -674,7 +729,8 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
 #pragma unroll
     for (int q = 0; q < QE; q++) {
       if (eoff[q] < 0) continue;
-      const int e = vt + q * NT;
+      int e = vt + q * NT;
+      if (kRupd && q > 0) asm volatile("" : "+v"(e));  // (second voxels: addresses not kept over the loop)
       const int ej = e / EK, ek = e - ej * EK;
       T fb[3][4], ft[3][4];
       face_load(nxt, ej, ek, ft);
@@ -774,28 +830,36 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T>())) void k_tiled(Dims g, c
       if (owns) {
         gather(nj + 1, nk + 1, Au);
 #pragma unroll
-        for (int c = 0; c < 3; c++)
-          rb[(c * (TJ + 1) + nj + 1) * (TK + 1) + nk + 1] = pin.e0[c] - Au[c];
+        for (int c = 0; c < 3; c++) {
+          T *at = rb + part + (c * (TJ + 1) + nj + 1) * (TK + 1) + nk + 1;
+          *at = (kRupd ? *at : pin.e0[c]) - Au[c];
+        }
       }
       if (extra) {
-        gather(xa, xb, Au);
+        int x = tid;
+        if (kRupd) asm volatile("" : "+v"(x));  // (addresses not kept over the loop)
+        const int ya = x <= TK ? 0 : x - TK, yb = x <= TK ? x : 0;
+        gather(ya, yb, Au);
 #pragma unroll
-        for (int c = 0; c < 3; c++) rb[(c * (TJ + 1) + xa) * (TK + 1) + xb] = xin[c] - Au[c];
+        for (int c = 0; c < 3; c++) {
+          T *at = rb + part + (c * (TJ + 1) + ya) * (TK + 1) + yb;
+          *at = (kRupd ? *at : xin[c]) - Au[c];
+        }
       }
     } else if (owns) {
       T Au[3];
       gather(nj, nk, Au);
       if (a.nt)  // (one uniform branch per node, not per store)
-        epilogue<T, ST, EP, true>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
+        epilogue<T, ST, EP, true>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv, al);
       else
-        epilogue<T, ST, EP, false>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv);
+        epilogue<T, ST, EP, false>(a, pin, ti, c1, c2, off, V, (int)nown, Au, uo, dv, al);
     }
   }
   if constexpr (RS) {
     __syncthreads();
-    restrict_plane(iend - 1);
+    restrict_plane(iend - 1, !kRupd ? 0 : part == 0 ? 2 * RP : part - RP);
   }
-  if ((EP == EP_AX || EP == EP_RES || EP == EP_FIN1 || EP == EP_LASTD) && a.dot) {
+  if ((EP == EP_AX || EP == EP_RES || EP == EP_FIN1 || EP == EP_LASTD || kRupd) && a.dot) {
     const int pidx = chunk * tiles + tile;
     block_partial(a.red, a.slot, r, pidx, block_sum_n<NT>(dv.a));
     if (EP == EP_RES) {
@@ -924,6 +988,10 @@ void launch_tiled(int st, int ep, const Dims &g, int R, const T *E, const ModeCo
   GO(ST_PROLONG, EP_FIN1)
   GO(ST_DPROLONG, EP_CHEB0)
   GO(ST_DPROLONG, EP_FIN1)
+  if constexpr (sizeof(T) == 4) {
+    GO(ST_PUPDX, EP_AX)
+    GO(ST_RUPD, EP_PRE)
+  }
 #undef GO
   throw std::runtime_error("no operator kernel for this stage/epilogue pair");
 }

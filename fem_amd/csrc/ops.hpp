@@ -10,7 +10,15 @@
 //                                                coarse correction in one)
 //   ST_PUPD      u + beta u2                    (PCG direction p = z + beta p_old,
 //                                                beta per RHS from a device array)
-// (D enters as its precomputed inverse: no divisions in the kernels)
+//   ST_PUPDX     the same, and x += alpha u2 at the owned node: the solution
+//                update of the previous iteration, whose direction u2 is
+//   ST_RUPD      (u - alpha u2) * theta_inv / D (u = r, u2 = q = A p: the residual
+//                update r' = r - alpha q and the degree-1 pre-smoothing; pout = r',
+//                and with `dot` the FP64 partial of r'.r'; b is r' itself)
+// (D enters as its precomputed inverse: no divisions in the kernels.  beta of
+// ST_PUPDX and alpha of ST_RUPD are formed from the partials of the dot products
+// by every workgroup: a launch of their own costs about 5 us, 2% of a V-cycle
+// iteration on a 64^3 cell)
 // Epilogue at each owned node, with Au the operator result and u_own the
 // staged value there:
 //   EP_AX       y = Au            (optional FP64 partial of u . Au; with ST_PUPD,
@@ -37,7 +45,7 @@
 
 namespace femh {
 
-enum Stage : int { ST_PLAIN = 0, ST_DSCALE = 1, ST_PROLONG = 2, ST_PUPD = 3, ST_DPROLONG = 4 };
+enum Stage : int { ST_PLAIN = 0, ST_DSCALE = 1, ST_PROLONG = 2, ST_PUPD = 3, ST_DPROLONG = 4, ST_PUPDX = 5, ST_RUPD = 6 };
 enum Epi : int {
   EP_AX = 0,
   EP_RES = 1,
@@ -55,9 +63,10 @@ constexpr int kMaxCheb = 16;
 template <typename T>
 struct OpArgs {
   const T *u = nullptr;      // staged vector [R][3][V]
-  const T *u2 = nullptr;     // ST_PUPD: previous direction [R][3][V]
+  const T *u2 = nullptr;     // ST_PUPD, ST_PUPDX: previous direction; ST_RUPD: q [R][3][V]
   const double *beta = nullptr;  // ST_PUPD: per-RHS beta [R]
-  T *pout = nullptr;         // ST_PUPD: staged value written back (new direction)
+  double *alpha = nullptr;       // per-RHS alpha [R]: read by ST_PUPDX, written by ST_RUPD
+  T *pout = nullptr;         // ST_PUPD, ST_PUPDX: staged value written back (new direction); ST_RUPD: r'
   const T *xc = nullptr;     // ST_PROLONG, ST_DPROLONG: coarse vector [R][3][Vc]
   Dims gc{};                 // ST_PROLONG, ST_DPROLONG, fine EP_PRE: coarse dims
   const T *Dinv = nullptr;   // inverse diagonal [B][3][V]
@@ -73,6 +82,12 @@ struct OpArgs {
   int slot = 0;
   int dot = 0;               // EP_RES: r.r -> slot, b.x -> slot2, x.r -> slot3
   int slot2 = 0, slot3 = 0;
+  // ST_PUPDX's beta and ST_RUPD's alpha are quotients of two sums of partials,
+  // slot2 (np of them) over slot3 (np3); `record` (optional) takes the value at
+  // row cnt[r] - ST_PUPDX, cnt the iterations done per RHS
+  int np = 0, np3 = 0;
+  double *record = nullptr;
+  const int *cnt = nullptr;
   // Chebyshev coefficients of this launch, device memory [3][kMaxB]: 1/theta,
   // c1, c2 per sample (null where the variant uses none).  In device memory,
   // not in the arguments, so that a recorded launch sequence stays valid when

@@ -231,7 +231,8 @@ double tiled_alg_bytes(int st, int ep, const OpArgs<T> &a, double V, double sz, 
       if (in[i] == p) return;
     in[nin++] = p;
   };
-  if (st == ST_PUPD) add_in(a.u2);
+  if (st == ST_PUPD || st == ST_PUPDX || st == ST_RUPD) add_in(a.u2);
+  if (st == ST_PUPDX) add_in(a.x);
   const bool step = ep == EP_STEP || ep == EP_LAST || ep == EP_LASTD;
   if (ep == EP_RES || ep == EP_PRE || ep == EP_CHEB0 || ep == EP_FIN1 || ep == EP_LASTD) add_in(a.b);
   if (step) {
@@ -239,12 +240,13 @@ double tiled_alg_bytes(int st, int ep, const OpArgs<T> &a, double V, double sz, 
     if (st != ST_DSCALE) add_in(a.xprev);
   }
   double vec = nin;
-  if (ep == EP_AX) vec += st == ST_PUPD ? 2 : 1;
+  if (ep == EP_AX) vec += st == ST_PUPDX ? 3 : st == ST_PUPD ? 2 : 1;
+  if (st == ST_RUPD) vec += 1;
   if (ep == EP_AXD || ep == EP_RES || ep == EP_FIN1 || ep == EP_LAST || ep == EP_LASTD) vec += 1;
   if (ep == EP_PRE) vec += 0.125;  // the restricted residual
   if (ep == EP_CHEB0 || ep == EP_STEP) vec += 3;
   if (st == ST_PROLONG || st == ST_DPROLONG) vec += 0.125;  // coarse correction, 1/8 of the nodes
-  const bool usesD = st == ST_DSCALE || st == ST_DPROLONG || ep == EP_CHEB0 || ep == EP_FIN1 || step || ep == EP_AXD;
+  const bool usesD = st == ST_RUPD || st == ST_DSCALE || st == ST_DPROLONG || ep == EP_CHEB0 || ep == EP_FIN1 || step || ep == EP_AXD;
   return V * (3.0 * sz * Rn * vec + ns * sz * (usesD ? 4.0 : 1.0));
 }
 
@@ -814,6 +816,13 @@ bool Context::vcycle(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_
     }
     launch_restrict<T>(L.g, C.g, R, L.r.template as<T>(), C.b.template as<T>(), act_, stream, xfer_planes(l));
   }
+  return coarse_post<T>(h, l, bb, xx, act_, dot_slot);
+}
+
+// the rest of a cycle once the coarse right-hand side is there
+template <typename T>
+bool Context::coarse_post(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_, int dot_slot) {
+  Level<T> &C = h.lv[l + 1];
   vcycle<T>(h, l + 1, C.b.template as<T>(), C.x.template as<T>(), act_, -1);
   return post_smooth<T>(h, l, bb, xx, act_, dot_slot);
 }
@@ -875,16 +884,31 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // ping-ponging p between pv and a second buffer since neighbours still
   // read the old direction.  beta comes from a one-block-per-RHS kernel.
   const bool fuse_p = o.apply_kernel != 1;
+  // Degree-1 smoothing in FP32: the updates ride along too.  r -= alpha q runs
+  // inside the pre-smoothing launch (ping-ponging r with the fine level's
+  // residual buffer, which that cycle leaves free), and x += alpha p inside the
+  // next iteration's A p launch, with one pass for every right-hand side's last
+  // update at the end.  As a pass of its own the update moves six vectors; here
+  // it adds two to each of the two launches.  Taken where a vector is larger than
+  // the 256 MB last-level cache, so that the six come from HBM (the solves with
+  // and without: 48 cells of 64^3 in batches of 16, 66.7 -> 63.1 ms; 8 cells of
+  // 96^3 with their gradient, 92.1 -> 90.7); below that the pass finds them in
+  // the cache and costs what the longer launches do (8 cells of 48^3, one of
+  // 128^3, one of 64^3 in either precision: within 1%).
+  const bool fuse_r = sizeof(T) == 4 && fuse_p && !jac && o.nu1 == 1 && o.nu2 == 1 &&
+                      field_bytes(g, nb, sizeof(T)) > (size_t)256 << 20;
+  T *rcur = rv, *rnxt = fuse_r ? h.lv[0].r.template as<T>() : nullptr;
   T *pcur = pv, *pnxt = nullptr;
   if (fuse_p) {
     DBuf &alt = sizeof(T) == 8 ? palt : palt32;
     if (!alt.p) alt.alloc(field_bytes(g, B, sizeof(T)));
-    if (!beta_d.p) beta_d.alloc(sizeof(double) * kMaxR);
+    if (!beta_d.p) beta_d.alloc(sizeof(double) * 2 * kMaxR);
     pnxt = alt.template as<T>();
     launch_beta(R, S_RZ0, S_RZ0, 1, ap, red, np_rz, beta_d.as<double>(), stream);
   } else {
     launch_p_update<T>(V, R, pv, zv, S_RZ0, S_RZ0, 1, ap, red, np_rz, stream);
   }
+  double *alpha_d = beta_d.p ? beta_d.as<double>() + kMaxR : nullptr;
   // Per-RHS iteration state on the device: iterations done, relative
   // residual, state (1 converged, 2 non-finite), and |b|^2.  The convergence
   // test runs on the device after every update, so an iteration is a fixed
@@ -910,10 +934,44 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
       a.red = red;
       a.slot = S_PQ;
       a.dot = 1;
-      op<T>(h, 0, ST_PUPD, EP_AX, a);
+      a.alpha = alpha_d;
+      a.x = xv;
+      a.slot2 = rzc;
+      a.slot3 = rzn;  // (the last iteration's r . z)
+      a.np = a.np3 = np_rz;
+      a.record = lz_beta;
+      a.cnt = cnt;
+      op<T>(h, 0, fuse_r && !first ? ST_PUPDX : ST_PUPD, EP_AX, a);
       std::swap(pcur, pnxt);
     } else {
       apply<T>(h, 0, pv, qv, nullptr, 0, ap, &red, S_PQ);
+    }
+    if (fuse_r) {
+      OpArgs<T> a;
+      a.act = ap;
+      a.u = rcur;
+      a.u2 = qv;
+      a.alpha = alpha_d;
+      a.pout = rnxt;
+      a.b = rcur;
+      a.y = h.lv[1].b.template as<T>();
+      a.gc = h.lv[1].g;
+      a.red = red;
+      a.slot = S_RR;
+      a.dot = 1;
+      a.slot2 = rzc;
+      a.np = np_rz;
+      a.slot3 = S_PQ;
+      a.np3 = apply_parts((int)sizeof(T));
+      a.record = lz_alpha;
+      a.cnt = cnt;
+      set_cheb(h, 0, a, 0, o.cheby_ratio);
+      op<T>(h, 0, ST_RUPD, EP_PRE, a);
+      std::swap(rcur, rnxt);
+      launch_pcg_check(R, apw, red, tiled_parts(g, R, shape_fine, (int)sizeof(T), true), bb_d, tol, cnt, relres_d, pst,
+                       stream);
+      coarse_post<T>(h, 0, rcur, zv, ap, rzn);
+      return;
     }
     launch_pcg_update<T>(V, R, xv, rv, pcur, qv, jac ? D0 : nullptr, zv, rzc, rzn, ap, red, apply_parts((int)sizeof(T)), np_rz,
                          stream, lz_alpha, cnt);
@@ -1018,8 +1076,9 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     live_rhs = q;
     shape_fine = tiled_sparse_shape(g, R, q, restore.shape, (int)sizeof(T));
     np_rz = rz_parts(h);
-    // r . z of the last iteration, in the old launch's partials, as one partial
-    launch_collapse(R, (it & 1) ? S_RZ1 : S_RZ0, red, np_old, np_rz, stream);
+    // r . z of the last two iterations, in the old launch's partials, as one partial
+    launch_collapse(R, S_RZ0, red, np_old, np_rz, stream);
+    launch_collapse(R, S_RZ1, red, np_old, np_rz, stream);
     FEMH_HIP(hipGetLastError());
     if (graphs && max_iter - it >= per_replay) record();
   };
@@ -1039,6 +1098,9 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // results of the run: iterations and residual per right-hand side, and which
   // are left (not converged within max_iter)
   if (live || max_iter == 1) poll();
+  if constexpr (sizeof(T) == 4) {
+    if (fuse_r) launch_x_last(V, R, xv, pv, palt32.as<float>(), alpha_d, cnt, stream);
+  }
   for (int t = 0; t < R; t++) {
     if (!active[t]) continue;
     iters[t] = hcnt[t];

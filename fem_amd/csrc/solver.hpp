@@ -143,7 +143,7 @@ struct Context {
   DBuf xw;          // warm start: previous fields [R][3][V] (FP64)
   DBuf dx, dq;      // mixed precision: FP64 fallback correction and PCG scratch
   DBuf palt, palt32;  // PCG: second direction buffer of the fused direction update
-  DBuf beta_d;        // PCG: per-RHS beta [kMaxR] (double)
+  DBuf beta_d;        // PCG: per-RHS beta, then alpha ([kMaxR] doubles each)
   std::vector<int> fallback_;  // per sample: finished in FP64 this call
   // Lanczos record of the mixed path's correction sweeps: alpha and beta of
   // every PCG iteration and right-hand side ([kInnerMaxIter][kMaxR] each);
@@ -262,6 +262,8 @@ struct Context {
              const Reduce *red, int slot);
   template <typename T>
   void pre_fine(Hierarchy<T> &h, const T *b, const int *act_);
+  template <typename T>
+  bool coarse_post(Hierarchy<T> &h, int l, const T *b, T *x, const int *act_, int dot_slot);
   template <typename T>
   bool post_smooth(Hierarchy<T> &h, int l, const T *b, T *x, const int *act_, int dot_slot);
   template <typename T>
