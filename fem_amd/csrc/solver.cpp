@@ -1056,7 +1056,10 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // cell left: 55-70 us a fine launch, and it was left for 400 of 470
   // iterations).  From kSparseAfter iterations on, the launches are sized for
   // the next of R/4, R/16, .. that covers those left.  Solves of ordinary
-  // length never get there, so they pay no second recording.
+  // length never get there, so they pay no second recording.  The launch shape
+  // sets the order of the dot partials, so the sizes change after fixed
+  // numbers of iterations only (25, 29, ..), each of which a replay and a
+  // kernel-by-kernel run look at alike, whatever check_every says.
   struct Restore {
     Context &c;
     int shape;
@@ -1066,8 +1069,9 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     }
   } restore{*this, shape_fine};
   constexpr int kSparseAfter = 24;
+  auto sizing = [&]() { return !jac && o.apply_kernel != 1 && it > kSparseAfter && it % 4 == 1; };
   auto resize = [&]() {
-    if (jac || o.apply_kernel == 1 || it < kSparseAfter || !live) return;
+    if (!sizing()) return;
     int q = live_rhs > 0 ? live_rhs : R;
     const int was = q;
     while (q / 4 >= nlive) q /= 4;
@@ -1093,7 +1097,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
     iteration(it & 1, false);
     it++;
     const int every = jac ? std::max(o.check_every, std::min(8, it / 8)) : o.check_every;
-    if (it % std::max(every, 1) == 0 || it == max_iter) live = poll();
+    if (it % std::max(every, 1) == 0 || it == max_iter || sizing()) live = poll();
   }
   // results of the run: iterations and residual per right-hand side, and which
   // are left (not converged within max_iter)

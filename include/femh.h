@@ -99,12 +99,20 @@ typedef struct femh_opts {
   int precision;        /* femh_precision */
   double ch_tol;        /* mixed: stop when the estimated relative C_H error of
                            every load case is below this (0 = use tol only) */
-  int check_every;      /* iterations between host convergence checks */
+  int check_every;      /* without `graph`: iterations between host convergence checks.
+                           Jacobi solves look less often (every eighth of the
+                           iterations done, up to every 8), multigrid solves also after
+                           iterations 25, 29, ..; results do not depend on it */
   int device;           /* HIP device ordinal */
   double inner_tol;     /* mixed: relative tolerance of each FP32 correction solve */
   int max_outer;        /* mixed: refinement sweep cap */
   int apply_kernel;     /* fine-grid operator: 0 tiled cube-mode (default), 1 dense gather */
-  int batch;            /* samples solved together per launch sequence (1..16) */
+  int batch;            /* samples solved together per launch sequence (1..16).  A
+                           multigrid solve that is down to a quarter of its load cases
+                           after 25 iterations sizes its launches for those left, which
+                           moves the order of their dot-product partial sums: the
+                           rounding of a slow cell's result depends on when the other
+                           cells of its batch converge */
   int coarse_nu;        /* smoothing degree (pre and post) on the coarse levels; 0: nu1/nu2
                            (default 3: coarse sweeps are cheap and save fine ones) */
   int warm_start;       /* 1: start each sample slot from the fields of the previous
@@ -141,10 +149,11 @@ typedef struct femh_opts {
                            each on its own sub-context and stream (0 = 8).  1 runs the
                            batches one after another on one thread */
   int graph;            /* 1 (default): PCG iterations run as a recorded launch sequence
-                           (hipGraph) of two iterations, replayed until every load case
-                           converged; the convergence test runs on the device and the
-                           host looks at it once per replay.  0: the same iterations
-                           launched one kernel at a time.  Results are the same */
+                           (hipGraph) of two iterations (eight with Jacobi), replayed
+                           until every load case converged; the convergence test runs
+                           on the device and the host looks at it once per replay.
+                           0: the same iterations launched one kernel at a time.
+                           Results are the same */
   int adapt_inner;      /* mixed with ch_tol > 0: 1 (default): a correction sweep after the
                            first stops at the residual reduction its cell's estimate
                            needs, 0.5 sqrt(ch_tol / estimate) clamped to [inner_tol, 0.1],
