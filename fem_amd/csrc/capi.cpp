@@ -418,6 +418,7 @@ int femh_prepare(femh_ctx *ctx, const double *E) {
     ctx->c->load(E, 1, false, true);
     ctx->c->build_hierarchy();
     ctx->c->check_setup();
+    ctx->c->h64.ready = true;
   });
 }
 

@@ -210,7 +210,7 @@ void Context::load(const double *src, int n, bool device_src, bool modulus) {
                     o.penal, stream);
   FEMH_HIP(hipGetLastError());
   modulus_input = modulus;
-  h64.ready = h32.ready = false;
+  h64.ready = false;
   have_fields = false;
 }
 
@@ -352,9 +352,8 @@ void Context::apply(Hierarchy<T> &h, int l, const T *u, T *y, const T *bb, int m
 
 // ---------------------------------------------------------------------------
 // hierarchy
-template <typename T>
-void Context::build_levels(Hierarchy<T> &h) {
-  // level dimensions: halve while every dimension is even and >= 4
+// level dimensions: halve while every dimension is even and >= 4
+std::vector<Dims> Context::level_dims() const {
   std::vector<Dims> dims{g};
   int maxL = (o.precond == FEMH_PRECOND_MG) ? (o.levels > 0 ? o.levels : 32) : 1;
   while ((int)dims.size() < maxL) {
@@ -364,6 +363,12 @@ void Context::build_levels(Hierarchy<T> &h) {
     c.V = c.nx * c.ny * c.nz;
     dims.push_back(c);
   }
+  return dims;
+}
+
+template <typename T>
+void Context::build_levels(Hierarchy<T> &h) {
+  const std::vector<Dims> dims = level_dims();
   h.lv.resize(dims.size());
   for (size_t l = 0; l < dims.size(); l++) {
     Level<T> &L = h.lv[l];
@@ -534,10 +539,21 @@ std::mutex g_tune_mu;
 std::map<std::array<int, 7>, std::vector<int>> g_tuned;
 }  // namespace
 
+static std::array<int, 7> tune_key(const Context &c, int sz, int levels) {
+  return {c.g.nx, c.g.ny, c.g.nz, c.R, sz, levels, c.o.apply_kernel};
+}
+
+// this call's build_hierarchy will time launch shapes
+bool Context::will_tune() const {
+  if (!o.autotune) return false;
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  return !g_tuned.count(tune_key(*this, o.precision == FEMH_MIXED ? 4 : 8, (int)level_dims().size()));
+}
+
 template <typename T>
 void Context::autotune(Hierarchy<T> &h) {
   const int L = (int)h.lv.size();
-  const std::array<int, 7> key{g.nx, g.ny, g.nz, R, (int)sizeof(T), L, o.apply_kernel};
+  const std::array<int, 7> key = tune_key(*this, (int)sizeof(T), L);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(key);
@@ -657,9 +673,7 @@ void Context::build_hierarchy() {
       estimate_lmax(h32);
     }
     FEMH_HIP(hipGetLastError());
-    h32.ready = true;
   }
-  h64.ready = true;
 }
 
 void Context::ensure_h64_ops() {
@@ -1235,16 +1249,30 @@ void Context::homogenize(double *C, femh_stats *st) {
   if (timed) FEMH_HIP(hipEventRecord(ev[0], stream));
   have_fields = false;
   // The moduli are checked with the set-up's other results, in one wait at its
-  // end: no kernel's indexing or trip count depends on their values.
+  // end: no kernel's indexing or trip count depends on their values.  (Before
+  // the set-up where it would time launch shapes: those of a refused cell are
+  // not kept.)  The hierarchy counts as built once everything has passed.
   // cubic structure: a cell takes the two-solve path only if its moduli are
   // invariant under the axis swaps (counted on the device); other cells of
   // the batch are solved with all six load cases
   const bool cubic = o.structure == FEMH_STRUCT_CUBIC;
   std::vector<double> mst(4 * nb);
   std::vector<char> cubic_ok(nb, 0);
+  auto check_moduli = [&]() {
+    for (int s = 0; s < nb; s++) {
+      if (mst[3 * s + 1] > 0) throw Error(FEMH_NONFINITE, "non-finite modulus");
+      if (mst[3 * s + 2] > 0) throw Error(FEMH_BAD_ARG, "negative modulus");
+      if (!(mst[3 * s] > 0)) throw Error(FEMH_BAD_ARG, "all-void cell (every modulus is zero)");
+    }
+  };
   {
     const int np = launch_modulus_stats(g.V, nb, E64.as<double>(), red, stream, cubic ? g.nx : 0);
-    launch_finalize(red, S_AUX, (cubic ? 4 : 3) * nb, np, stream);
+    if (will_tune()) {
+      read_scalars(S_AUX, mst.data(), (cubic ? 4 : 3) * nb, np);
+      check_moduli();
+    } else {
+      launch_finalize(red, S_AUX, (cubic ? 4 : 3) * nb, np, stream);
+    }
   }
   std::vector<int> all(R, 1);
   set_act(A_ALL, all);
@@ -1259,12 +1287,9 @@ void Context::homogenize(double *C, femh_stats *st) {
   std::vector<double> setup(2 * kSlotWidth);
   check_setup(setup.data());
   std::copy(setup.begin() + kSlotWidth, setup.begin() + kSlotWidth + mst.size(), mst.begin());
-  for (int s = 0; s < nb; s++) {
-    if (mst[3 * s + 1] > 0) throw Error(FEMH_NONFINITE, "non-finite modulus");
-    if (mst[3 * s + 2] > 0) throw Error(FEMH_BAD_ARG, "negative modulus");
-    if (!(mst[3 * s] > 0)) throw Error(FEMH_BAD_ARG, "all-void cell (every modulus is zero)");
-  }
+  check_moduli();
   if (o.precond == FEMH_PRECOND_MG && nlevels > 1) raise_setup(setup.data());
+  h64.ready = true;
   if (cubic)
     for (int s = 0; s < nb; s++) cubic_ok[s] = mst[3 * nb + s] == 0.0;
   std::vector<double> bb(setup.begin(), setup.begin() + R);

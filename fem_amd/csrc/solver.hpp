@@ -101,7 +101,7 @@ struct Hierarchy {
   DBuf cheb;
   int cheb_steps = 0;
   int ndense = 0;
-  bool ready = false;
+  bool ready = false;  // (h64: built, and the cell passed every check)
 };
 
 // Chebyshev interval [lmax / ratio, lmax] of the iterative coarsest solve
@@ -193,6 +193,7 @@ struct Context {
   int live_rhs = 0;
   int live_cells() const { return live_rhs > 0 && live_rhs < nb ? live_rhs : nb; }
   int xfer_planes(int l) const { return live_rhs > 0 ? 1 : xfer_shape(l); }
+  bool will_tune() const;
   template <typename T>
   void autotune(Hierarchy<T> &h);
 
@@ -251,6 +252,7 @@ struct Context {
  private:
   const int *actp(int slot) const { return act.as<int>() + slot * kMaxR; }
   void set_act(int slot, const std::vector<int> &v);
+  std::vector<Dims> level_dims() const;
   template <typename T>
   void build_levels(Hierarchy<T> &h);
   template <typename T>
