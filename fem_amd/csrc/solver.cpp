@@ -897,7 +897,12 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // inside the A p launch (staged on the fly, written back by the owner),
   // ping-ponging p between pv and a second buffer since neighbours still
   // read the old direction.  beta comes from a one-block-per-RHS kernel.
-  const bool fuse_p = o.apply_kernel != 1;
+  // A Jacobi solve, whose context may fill the device with little else than
+  // its vectors, takes a vector that idles meanwhile as the second buffer: an
+  // FP64 solve the right-hand side, which r has a copy of, an FP32 sweep of the
+  // mixed path an FP64 scratch vector.  The mixed path's FP64 fallback has none
+  // and updates the direction in a pass of its own.
+  const bool fuse_p = o.apply_kernel != 1 && !(jac && sizeof(T) == 8 && o.precision == FEMH_MIXED);
   // Degree-1 smoothing in FP32: the updates ride along too.  r -= alpha q runs
   // inside the pre-smoothing launch (ping-ponging r with the fine level's
   // residual buffer, which that cycle leaves free), and x += alpha p inside the
@@ -914,7 +919,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   T *rcur = rv, *rnxt = fuse_r ? h.lv[0].r.template as<T>() : nullptr;
   T *pcur = pv, *pnxt = nullptr;
   if (fuse_p) {
-    DBuf &alt = sizeof(T) == 8 ? palt : palt32;
+    DBuf &alt = jac ? (sizeof(T) == 8 ? b : p) : sizeof(T) == 8 ? palt : palt32;
     if (!alt.p) alt.alloc(field_bytes(g, B, sizeof(T)));
     if (!beta_d.p) beta_d.alloc(sizeof(double) * 2 * kMaxR);
     pnxt = alt.template as<T>();

@@ -142,7 +142,7 @@ struct Context {
   int prev_nb = 0;  // samples of the last successful call (warm start source)
   DBuf xw;          // warm start: previous fields [R][3][V] (FP64)
   DBuf dx, dq;      // mixed precision: FP64 fallback correction and PCG scratch
-  DBuf palt, palt32;  // PCG: second direction buffer of the fused direction update
+  DBuf palt, palt32;  // multigrid PCG: second direction buffer of the fused direction update
   DBuf beta_d;        // PCG: per-RHS beta, then alpha ([kMaxR] doubles each)
   std::vector<int> fallback_;  // per sample: finished in FP64 this call
   // Lanczos record of the mixed path's correction sweeps: alpha and beta of
