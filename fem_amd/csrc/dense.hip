@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kBlock) void k_chol_backward(int n, const double *_
   }
 }
 
-size_t dense_work_doubles(int n, int B) { return (size_t)3 * n * n * B; }
+size_t dense_work_doubles(int n, int nb) { return n <= kSmallDense ? 0 : (size_t)3 * n * n * nb; }
 
 template <typename T>
 void launch_dense_inverse(const Dims &g, int nb, const T *S, double *work, T *Ainv, int *bad, hipStream_t s) {

@@ -152,8 +152,9 @@ void launch_prolong_add(Dims fine, Dims coarse, int R, const T *ec, T *ef, const
 // Ainv[s] = (A + (mean diagonal / V) Z Z^T)^-1 of each sample's operator with
 // stencil S on grid g (Z the three constant fields), formed in FP64;
 // bad[s] = 1 where a pivot was not positive (dense.hip).  work holds
-// dense_work_doubles(3 g.V, samples) doubles.
-size_t dense_work_doubles(int n, int B);
+// dense_work_doubles(3 g.V, nb) doubles (none for the small matrices, which
+// stay in LDS).
+size_t dense_work_doubles(int n, int nb);
 template <typename T>
 void launch_dense_inverse(const Dims &g, int nb, const T *S, double *work, T *Ainv, int *bad, hipStream_t s);
 // dense coarsest solve: x = Ainv[s] b for each RHS (n = 3*V_coarsest)

@@ -494,7 +494,7 @@ void Context::dense_coarse(Hierarchy<T> &h) {
   h.ndense = 0;
   if (n > 648 || h.lv.size() < 2) return;
   h.Ainv.alloc(sizeof(T) * (size_t)n * n * B);
-  dense_work.alloc(sizeof(double) * dense_work_doubles(n, B));
+  dense_work.alloc(sizeof(double) * dense_work_doubles(n, nb));  // (of the cells at hand, not of the capacity)
   dense_bad.alloc(sizeof(int) * kMaxB);
   launch_dense_inverse<T>(L.g, nb, L.S.template as<T>(), dense_work.as<double>(), h.Ainv.template as<T>(),
                           dense_bad.as<int>(), stream);

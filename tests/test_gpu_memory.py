@@ -28,3 +28,16 @@ def test_jacobi_call_adds_no_vector(precision):
     got = growth(h, E)
     h.close()
     assert levels / 2 < got < levels + (64 << 20), (got, levels)
+
+
+def test_dense_inverse_workspace_is_of_the_cells_at_hand():
+    """648 coarsest unknowns, one cell in a context for 16: three FP64 matrices
+    (10 MB) of workspace, not 16 times three (161 MB)."""
+    n, batch, V = 12, 16, 12 ** 3 + 6 ** 3
+    E = W.binary_modulus(W.binary_cube(n, 1, p=0.7), 1.0, 0.1)[None]
+    h = Homogenizer((n, n, n), nu=0.3, interp="modulus", levels=2, batch=batch)
+    got = growth(h, E)
+    h.close()
+    vectors = (7 * V + n ** 3) * 18 * batch * 8  # seven per level, the second direction
+    operators = ((6 * V + 243 * 6 ** 3 + n ** 3) * batch + 648 ** 2 * batch) * 8
+    assert got < vectors + operators + 3 * 648 ** 2 * 8 + (64 << 20), (got, vectors, operators)
