@@ -529,7 +529,8 @@ void Context::build_ops(Hierarchy<T> &h) {
 // Launch-shape autotuner.  For each (grid, right-hand sides, precision,
 // levels) it times the fine operator (y = A u on every right-hand side) for a
 // few node-plane depths per workgroup, and the grid transfers (restriction
-// plus prolongation) of every level pair for a few planes per thread, on the
+// plus prolongation) of every pair of coarse levels for a few planes per thread
+// (the fine level's run inside its launches), on the
 // context's own buffers and stream, and keeps the fastest.  A candidate
 // within 2% of the built-in choice leaves the built-in choice in place.
 // Results are cached for the process, so later contexts of the same shape
@@ -621,7 +622,7 @@ void Context::autotune(Hierarchy<T> &h) {
     }
     shape_fine = pick(cand, t);
   }
-  for (int l = 0; l + 1 < L; l++) {
+  for (int l = 1; l + 1 < L; l++) {
     Level<T> &F = h.lv[l], &C = h.lv[l + 1];
     std::vector<int> cand{0, 1, 2, 4, 8};
     std::vector<double> t;

@@ -175,7 +175,7 @@ struct Context {
   }
   long long xfer_hash() const {
     long long hsh = 1469598103934665603ll;
-    for (int v : shape_xfer) hsh = (hsh ^ v) * 1099511628211ll;
+    for (size_t l = 1; l < shape_xfer.size(); l++) hsh = (hsh ^ shape_xfer[l]) * 1099511628211ll;
     return hsh;
   }
   template <typename T>
@@ -184,7 +184,8 @@ struct Context {
   int nlevels = 1;
   // launch shapes (0: the built-in choice): node planes per workgroup of the
   // fine operator, coarse planes per thread of the transfers between level l
-  // and l + 1; set by the autotuner
+  // and l + 1 (entry 0 is not used: the fine level's run inside its launches);
+  // set by the autotuner
   int shape_fine = 0;
   std::vector<int> shape_xfer;
   int xfer_shape(int l) const { return l < (int)shape_xfer.size() ? shape_xfer[l] : 0; }

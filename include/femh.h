@@ -129,8 +129,8 @@ typedef struct femh_opts {
                            (NumericalCoarseningUsingMultiGrid.cpp:275-282) makes the
                            same two solves */
   int autotune;         /* 1: before the first solve of each (grid, batch, precision)
-                           shape in the process, time the fine operator and the grid
-                           transfers for a few launch shapes (tile of node columns
+                           shape in the process, time the fine operator and the coarse
+                           grid transfers for a few launch shapes (tile of node columns
                            and node planes per workgroup, planes per thread) and
                            keep the fastest; the
                            choice is cached for the process.  The fine-operator
@@ -278,8 +278,9 @@ int femh_thermal_expansion(struct femh_ctx *ctx, const double *alpha, double *be
  * shapes[0] = the fine operator's shape (bits 0-7 node planes per workgroup,
  * bits 8-15 the tile of owned node columns per workgroup: 1 = 16 x 16,
  * 2 = 8 x 32, 3 = 16 x 32), shapes[1 + l] =
- * coarse planes per thread of the transfers between levels l and l + 1.
- * Writes at most n values; returns their count (levels) or a negative status.
+ * coarse planes per thread of the transfers between levels l and l + 1
+ * (shapes[1] is accepted and reported but has no effect: the transfers of the
+ * fine level run inside its operator launches).  Writes at most n values; returns their count (levels) or a negative status.
  * No counterpart in the reference, whose CPU loops have no launch shapes. */
 int femh_launch_shapes(struct femh_ctx *ctx, int *shapes, int n);
 

@@ -52,3 +52,20 @@ def test_autotuned_mixed_uneven_batch_within_1e6():
         C64, _ = h.homogenize_modulus(g)
         h.close()
         assert rel(C[s], C64) <= 1e-6, (s, g.shape, rel(C[s], C64))
+
+
+def test_fine_level_transfers_are_not_tuned():
+    # (they run inside the fine operator's launches: no shape of theirs has an effect)
+    n, batch = 64, 8
+    E = np.stack([W.simp_modulus(W.simp_density(n, s, 4.0)) for s in range(batch)])
+    kw = dict(nu=0.3, tol=1e-8, batch=batch, precision="mixed", ch_tol=1e-6)
+    h = Homogenizer((n, n, n), autotune=True, **kw)
+    h.homogenize_many(E, modulus=True)
+    assert h.launch_shapes()[1] == 0
+    h.close()
+    h = Homogenizer((n, n, n), **kw)
+    C0, _ = h.homogenize_many(E, modulus=True)
+    h.set_launch_shapes([0, 4])
+    C1, _ = h.homogenize_many(E, modulus=True)
+    assert h.launch_shapes()[1] == 4 and np.array_equal(C0, C1)
+    h.close()
