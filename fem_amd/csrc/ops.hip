@@ -273,11 +273,26 @@ __device__ __forceinline__ int xcd_order(int b, int n) {
 //  * spread: eighth of the units, cell, unit within the eighth, inner: every
 //    XCD gets an eighth of every cell (that launch: 24 us).
 // Spread is taken for launches sized for a few remaining right-hand sides
-// (live_rhs), and whenever the units divide by eight, so that an eighth is a
-// block of whole neighbours and cells that converge early leave no XCD idle
-// (48 cells of 64^3: 77.1 -> 75.3 ms).  Elsewhere it costs more halo traffic
-// than it balances (40^3 in FP64, 18 units: 33.2 -> 39.3 ms).
-static inline int spread_rule(int sparse, int units) { return sparse || units % 8 == 0; }
+// (live_rhs), and where every eighth is the same number of equal units and
+// large enough for neighbours to share their halos:
+//  * the units divide by eight; otherwise an XCD has up to twice another's work
+//    (40^3 in FP64, 18 units: 33.2 -> 39.3 ms);
+//  * fine launches: chunks of one length.  A shorter last chunk lies on the
+//    same XCDs for every cell (chunks of 32 and 8 planes, 16 cells of 40 x 64 x
+//    96 in mixed precision: 1.19 times the time; 24^3, 16 + 8: 1.13 in FP64;
+//    48 x 64 x 64, 32 + 16: 1.09; 56^3, 32 + 24: 1.05);
+//  * at least two fine units per eighth (one: 32^3, 16 cells: 1.06) and eight
+//    stencil units (two, the level of 32^3: 1.02; ten or twelve, the levels of
+//    40^3 and 48^3: 1.00-1.01 where all cells take as long, but 0.98 in an uneven
+//    batch of 64 binary cells, whose cells converge one after the other).
+// Within these it cost no more than the 1% to which runs agree, but for 1.6%
+// on 4 cells of 32 x 64 x 128 in mixed precision; 64^3 0.97-0.99, 80^3 and 96^3
+// 0.99, 64 x 96 x 64 0.94, 128 x 64 x 64 0.95-0.98, 32 x 64 x 128 in FP64 0.95 of
+// the time.
+constexpr int kSpreadFine = 16, kSpreadStencil = 64;  // least units
+static inline int spread_rule(int sparse, int units, int least, bool equal) {
+  return sparse || (units % 8 == 0 && units >= least && equal);
+}
 struct WorkId {
   int cell, unit, inner;
 };
@@ -912,7 +927,7 @@ static void tiled_go(const Dims &g, int R, const T *E, const ModeC<T> &mc, const
   // vector still in the 256 MB last-level cache (one 64^3 cell in FP64, 38
   // MB, solves as fast either way)
   OpArgs<T> an = a;
-  an.spread = spread_rule(a.spread, tiles * chunks);
+  an.spread = spread_rule(a.spread, tiles * chunks, kSpreadFine, g.nx % TI == 0);
   an.nt = (size_t)R * 3 * (size_t)g.V * sizeof(T) >= ((size_t)128 << 20) ? 1 : 0;
   if (R % kRHS) throw std::runtime_error("right-hand sides must come in groups of six");
   if (fused &&
@@ -1367,8 +1382,12 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   // per CU.  One cell, and FP64 in general, take it with three load cases per
   // workgroup from 192 workgroups on: the nine-wave split kernel below re-reads
   // the row for every load case (a smoothing step of one cell: FP32 32^3, 17.3
-  // -> 9.7 us; FP64 30 x 22 x 26, 240 workgroups, 30.8 -> 13.6 us).  The power
-  // iteration runs one load case.
+  // -> 9.7 us; FP64 30 x 22 x 26, 240 workgroups, 30.8 -> 13.6 us).  Around that
+  // line, whole solves of one cell with 16-wide levels, split -> one-plane, FP64
+  // and mixed: 96 workgroups 8.9 -> 9.2 and 4.1 -> 4.3 ms, 128 9.3 -> 9.1 and
+  // 3.85 -> 3.91 (with 32 x 16 planes 8.5 -> 8.7 and 3.5 -> 3.65), 160 11.0 ->
+  // 10.2 and 4.3 -> 4.2, 192 13.7 -> 12.2 and 5.0 -> 4.8, 256 17.5 -> 14.9 and
+  // 6.0 -> 5.4.  The power iteration runs one load case.
   const int tiles_k = (g.nz + kTile - 1) / kTile, tiles_j = (g.ny + kTile - 1) / kTile;
   const long units = (long)tiles_j * tiles_k * g.nx;
   // (and a sample's stencil addressable by a buffer resource: < 2 GiB)
@@ -1389,7 +1408,7 @@ void launch_stencil(int st, int ep, const Dims &g, int R, const T *S, const OpAr
   // step; three per workgroup, 128 left: 6.6 us)
   const int nr = R % kRHS == 0 && (long)split_blocks * cells * kRHS >= 256 ? 2 : 1;
   OpArgs<T> an = a;
-  an.spread = spread_rule(a.spread, (int)units);
+  an.spread = spread_rule(a.spread, (int)units, kSpreadStencil, true);
 #define PLANE(S_, E_, NG_, SYM_, GRID_)                                                             \
   hipLaunchKernelGGL((k_stencil_plane<T, S_, E_, NG_, SYM_>), dim3(GRID_), dim3(kBlock), 0, s, g, S, an, tiles_k, \
                      tiles_j *tiles_k)
