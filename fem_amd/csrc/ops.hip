@@ -335,8 +335,8 @@ __device__ __forceinline__ double bload(__amdgpu_buffer_rsrc_t r, unsigned voff,
 // vectors, and the launches around them one more each, at 4.2-4.6 of the 4.85
 // TB/s that a large copy reaches.  64^3, 16 cells in FP32: pre-smoothing 297 us
 // and restriction 92 us became one launch of 282 us, prolongation 106 us and
-// post-smoothing 227 us one of 285 us; these launches now keep the VALU 68% busy
-// (62% without a transfer), and that, not the vectors, is what bounds them.
+// post-smoothing 227 us one of 285 us; these launches keep the VALU 62-63% busy,
+// and that, not the vectors, is what bounds them.
 //  * RS (EP_PRE): the residual goes to the coarse right-hand side and never to
 //    memory.  The tile computes one more node row and column at its low j and
 //    k sides (and its chunk one more plane), so that every coarse node above
@@ -886,7 +886,9 @@ __global__ __launch_bounds__(TJ * TK, (tiled_waves<T, ST, TJ * TK>())) void k_ti
 
 // Workgroups of the fine operator resident on the device at once for an
 // element size and tile: the occupancy of a representative variant (a
-// Chebyshev step) times the CU count, looked up once per process.
+// Chebyshev step) times the CU count, looked up once per process.  (The
+// variants with a grid transfer hold more LDS, so fewer of theirs may be: a
+// chunk length that gives the others one round can give them two.)
 template <typename T, int TJ, int TK>
 static int tiled_resident_of() {
   int per_cu = 0, dev = 0, cus = 0;

@@ -530,11 +530,10 @@ void Context::build_ops(Hierarchy<T> &h) {
 // levels) it times the fine operator (y = A u on every right-hand side) for a
 // few node-plane depths per workgroup, and the grid transfers (restriction
 // plus prolongation) of every pair of coarse levels for a few planes per thread
-// (the fine level's run inside its launches), on the
-// context's own buffers and stream, and keeps the fastest.  A candidate
-// within 2% of the built-in choice leaves the built-in choice in place.
-// Results are cached for the process, so later contexts of the same shape
-// take them without timing.
+// (the fine level's run inside its launches), on the context's own buffers and
+// stream, and keeps the fastest.  A candidate within 2% of the built-in choice
+// leaves the built-in choice in place.  Results are cached for the process, so
+// later contexts of the same shape take them without timing.
 namespace {
 std::mutex g_tune_mu;
 std::map<std::array<int, 7>, std::vector<int>> g_tuned;
@@ -754,7 +753,7 @@ void Context::pre_fine(Hierarchy<T> &h, const T *bb, const int *act_) {
 
 // The k = nu2 Chebyshev steps after the coarse correction x + P xc, on level l,
 // ending in xx.  The fine level stages the correction inside the first step;
-// the coarse levels add it in place first.  Returns true when the last launch
+// the coarse levels add it first, into xn.  Returns true when the last launch
 // also left the partials of b . x in dot_slot (fine level).
 template <typename T>
 bool Context::post_smooth(Hierarchy<T> &h, int l, const T *bb, T *xx, const int *act_, int dot_slot) {
@@ -1029,7 +1028,7 @@ void Context::pcg(Hierarchy<T> &h, const T *bvec, T *xv, T *rv, T *zv, T *pv, T 
   // Iterations 2k and 2k+1 use the same buffers and slots (ping-pong of the
   // direction and of the r.z parity), so with graphs on, the pair is
   // recorded once into a hipGraph and replayed; the host looks at the device
-  // state after every pair (or every check_every iterations without graphs).
+  // state after every replay (or every check_every iterations without graphs).
   // A Jacobi iteration is three short launches (about 20 us at 16^3), of which a
   // look at the state costs as much as one whole iteration, and an iteration of
   // converged right-hand sides is three launches that return at once: eight

@@ -159,8 +159,8 @@ struct Context {
   DBuf lm_part, lmax_d;
   DBuf dense_work, dense_bad;  // dense coarsest inverse: FP64 matrices and panels, per-sample failure flag
   DBuf ls_part, ls_h;  // device line search: per-cell block partials [n][kRedBlocks], steps [n]
-  // recorded PCG iteration pairs (hipGraph), keyed by everything their
-  // launches bake in: precision, right-hand sides, vector and hierarchy
+  // recorded PCG iterations (hipGraph: two, or eight with Jacobi), keyed by
+  // everything their launches bake in: precision, right-hand sides, vector and hierarchy
   // buffers, launch shapes, tolerance
   struct GraphKey {
     std::array<long long, 15> v{};

@@ -56,3 +56,19 @@ def test_noalloc_rejects_oversized_grid_and_other_solvers():
         homogenize_device_noalloc((8, 8, 8), d_rho.data_ptr(), d_C.data_ptr(), nu=NU, precond="mg")
     assert e.value.status == BAD_ARG
     assert float(d_C.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("shape", [(32, 32, 32), (2, 128, 128), (128, 16, 16)])
+def test_noalloc_takes_the_largest_grids(shape):
+    torch = pytest.importorskip("torch")
+    dev = torch.device("cuda:0")
+    assert int(np.prod(shape)) == NOALLOC_MAX_VOXELS
+    kw = dict(nu=NU, penal=3.0, precond="jacobi", tol=1e-10, max_iter=20000)
+    d_rho = torch.from_numpy(W.simp_density(shape, 5, 2.0, rho_min=0.2)).to(dev)
+    d_C = torch.zeros((2, 36), dtype=torch.float64, device=dev)
+    st = homogenize_device_noalloc(shape, d_rho.data_ptr(), d_C[0].data_ptr(), **kw)
+    h = Homogenizer(shape, **kw)
+    ref = h.homogenize_device(d_rho.data_ptr(), d_C[1].data_ptr())
+    h.close()
+    C = d_C.cpu().numpy()
+    assert rel(C[0], C[1]) <= 1e-12 and st["iters"] == ref["iters"]
